@@ -160,285 +160,368 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
 // is the fp32-accumulated product the reference forms -- the order of the
 // fp32 additions differs (as it does in the VALU kernel), inside the same
 // summation bound.  A weight of +-inf would meet a zero part (inf * 0 = NaN
-// where the reference has +-inf): rows holding one are flagged while they
-// stream and recomputed with fp32 fused multiply-adds in the epilogue.
-//   * v_mfma_f32_16x16x32_bf16: A = 16 rows of W x 32 k (lane l: row l % 16,
-//     its 8 k of group l / 16, one 16-byte load), B = 32 k x 16 batch rows of
-//     one part (the same k per lane from LDS), D = 16 rows x 16 batch rows
-//     (lane l: batch row l % 16, rows 4 (l / 16) .. +3);
-//   * a workgroup of 8 waves owns LMM_ROWS = 256 rows of W (2 tiles of 16 per
-//     wave; two workgroups per CU, one loading while the other computes),
-//     walks k in chunks of LMM_KC: the chunk's activation parts of the
-//     batch tile (16 NT rows) in LDS, each wave's W loads for the chunk all in
-//     flight (8 per tile), three parts x NT MFMAs per 32 k and tile;
-//   * W is read once per batch tile of 16 NT rows; the activations once per
-//     workgroup.
+// where the reference has +-inf): a workgroup that saw one recomputes those
+// rows with fp32 fused multiply-adds before its epilogue.
+//
+//   * k_lmx_split writes the parts once per call into the sampler's
+//     workspace, in the order the matrix cores read them ("fragments": 16
+//     batch rows x 32 k of one part, lane l's 8 values at 16 l), so the GEMM
+//     moves them to LDS and reads them back without conversions or bank
+//     conflicts.  Converting inside the GEMM instead cost every workgroup
+//     the whole conversion again, and LDS writes of 2 bytes per lane.
+//   * v_mfma_f32_16x16x32_bf16: A = 16 rows of W x 32 k, B = 32 k x 16 batch
+//     rows of one part, D = 16 rows x 16 batch rows (lane l: batch row l %
+//     16, rows 4 (l / 16) .. +3).  The smallest part goes first.
+//   * A workgroup owns WR TR x 16 rows of W and WC TC x 16 batch rows; wave
+//     (wr, wc) TR x TC tiles of it.  k advances in stages of KS x 32, NS
+//     stages of LDS in a ring: W and parts come by LDS-direct 16-byte loads
+//     (global_load_lds_dwordx4) NS - 1 stages ahead, one barrier per stage,
+//     the loads spread between the stage's MFMAs.
+//   * KS = 2: one load instruction takes 8 rows x 128 bytes of W, whole
+//     cache lines (64-byte pieces, KS = 1, reach 4.0 TB/s at 16 batch rows
+//     where KS = 2 reaches 5.4); the 16-byte pieces of a row are rotated by
+//     XOR with the row in the source address so that the fragment reads do
+//     not meet in the banks.  The 256 x 256 tile's stage only fits with
+//     KS = 1; it is bound by the matrix cores, not by that.
+//   * Bounds: above about 64 batch rows the three parts' 6 V n B operations
+//     (1.3 PFLOP/s at 256 rows, against 1.65 for a large library bf16 product
+//     on the same card), below that one read of W.
+// Workgroups of one row tile (its batch blocks) are consecutive on one XCD,
+// so its L2 serves W to all but the first.
 // MODE 1 (argmax keys) as in k_lmhead.
 typedef __bf16 lm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float lm_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t lm_u32x4 __attribute__((ext_vector_type(4)));
-constexpr int LMM_WAVES = 8;
-constexpr int LMM_TILES = 2;                       // 16-row tiles per wave
-constexpr int LMM_ROWS = LMM_WAVES * LMM_TILES * 16;  // 256 (two workgroups per CU)
-constexpr int LMM_KC = 128;                        // k per LDS chunk
-constexpr int LMM_KS = LMM_KC / 32;                // MFMA k-steps per chunk
-constexpr int LMM_PAD = 8;                         // bf16 of padding per LDS row (banks)
-constexpr int LMM_RS = LMM_KC + LMM_PAD;           // LDS row stride in bf16
+typedef uint16_t lm_u16x2 __attribute__((ext_vector_type(2)));
+constexpr int LMX_FRAG = 512;  // bf16 of one fragment (16 x 32)
 
 __device__ __forceinline__ float lm_bf16_f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
-
-// A 16-byte load of 8 weights holds an infinite or NaN one.
-__device__ __forceinline__ bool lm_nonfinite8(const lm_u32x4 q) {
-  bool r = false;
-#pragma unroll
-  for (int c = 0; c < 4; c++)
-    r |= ((q[c] & 0x7f800000u) == 0x7f800000u) | ((q[c] & 0x7f80u) == 0x7f80u);
-  return r;
-}
 
 // Keys of the fused argmax spread over LMM_SLOTS slots per batch row (one
 // per workgroup index modulo LMM_SLOTS, each on its own cache line), so the
 // workgroups' atomics do not all meet on the batch's few words.
 constexpr int LMM_SLOTS = 16;
 
-// One chunk's activations: 16 NT batch rows x LMM_KC, loaded into registers
-// (XPT per thread), then split into the three bf16 parts in LDS.
-template <int NT>
-struct LmX {
-  static constexpr int XPT = 16 * NT * LMM_KC / (64 * LMM_WAVES);
-  float v[XPT];
-};
-
-template <int NT>
-__device__ __forceinline__ void lm_x_load(LmX<NT>& xr, const float* __restrict__ X, long ldx,
-                                          int nb, int n, int k0) {
+// The activations' three bf16 parts as fragments: part p of batch rows 16 ct
+// .. +15 and k 32 ks .. +31 at xp[((ks * ctt + ct) * 3 + p) * LMX_FRAG]
+// (zeros past nb and past n).  One wave per (ks, ct).
+__global__ __launch_bounds__(64) void k_lmx_split(const float* __restrict__ X, long ldx, int nb,
+                                                  int n, int ctt, uint16_t* __restrict__ xp) {
+  const int ks = blockIdx.x, ct = blockIdx.y, lane = threadIdx.x;
+  const int b = ct * 16 + (lane & 15), k0 = ks * 32 + 8 * (lane >> 4);
+  uint32_t h[3][4];
 #pragma unroll
-  for (int q = 0; q < LmX<NT>::XPT; q++) {
-    const int i = (int)threadIdx.x + q * 64 * LMM_WAVES;
-    const int b = i / LMM_KC, kk = i - b * LMM_KC;
-    xr.v[q] = b < nb && k0 + kk < n ? X[(size_t)b * ldx + k0 + kk] : 0.0f;
-  }
-}
-
-template <int NT>
-__device__ __forceinline__ void lm_x_store(const LmX<NT>& xr, uint16_t* xs) {
-#pragma unroll
-  for (int q = 0; q < LmX<NT>::XPT; q++) {
-    const int i = (int)threadIdx.x + q * 64 * LMM_WAVES;
-    const int b = i / LMM_KC, kk = i - b * LMM_KC;
-    const float x = xr.v[q];
+  for (int e = 0; e < 8; e++) {
+    const float x = b < nb && k0 + e < n ? X[(size_t)b * ldx + k0 + e] : 0.0f;
     const uint32_t ux = __float_as_uint(x);
     const bool fin = (ux & 0x7f800000u) != 0x7f800000u;
     // (a NaN whose payload sits in the low bits stays a NaN)
-    const uint16_t h0 = fin || !(ux & 0x7fffffu) ? (uint16_t)(ux >> 16) : (uint16_t)0x7fc0u;
-    const float r0 = fin ? x - lm_bf16_f(h0) : 0.0f;  // exact: x's low 16 significand bits
-    const uint16_t h1 = (uint16_t)(__float_as_uint(r0) >> 16);
-    const float r1 = r0 - lm_bf16_f(h1);  // exact: at most 8 significant bits left
-    const uint16_t h2 = (uint16_t)(__float_as_uint(r1) >> 16);
-    xs[(0 * 16 * NT + b) * LMM_RS + kk] = h0;
-    xs[(1 * 16 * NT + b) * LMM_RS + kk] = h1;
-    xs[(2 * 16 * NT + b) * LMM_RS + kk] = h2;
+    const uint32_t h0 = fin || !(ux & 0x7fffffu) ? ux >> 16 : 0x7fc0u;
+    const float r0 = fin ? x - __uint_as_float(h0 << 16) : 0.0f;  // exact: the low 16 bits
+    const uint32_t h1 = __float_as_uint(r0) >> 16;
+    const float r1 = r0 - __uint_as_float(h1 << 16);  // exact: at most 8 significant bits left
+    const uint32_t h2 = __float_as_uint(r1) >> 16;
+    const uint32_t hs[3] = {h0, h1, h2};
+#pragma unroll
+    for (int p = 0; p < 3; p++) h[p][e >> 1] = e & 1 ? h[p][e >> 1] | hs[p] << 16 : hs[p];
   }
+  uint16_t* o = xp + ((size_t)ks * ctt + ct) * 3 * LMX_FRAG + lane * 8;
+#pragma unroll
+  for (int p = 0; p < 3; p++)
+    *reinterpret_cast<lm_u32x4*>(o + p * LMX_FRAG) = lm_u32x4{h[p][0], h[p][1], h[p][2], h[p][3]};
 }
 
-__device__ __forceinline__ void lm_w_load(lm_u32x4 (&a)[LMM_TILES][LMM_KS],
-                                          const uint16_t* const (&wr)[LMM_TILES], int n, int k0,
-                                          int g) {
-#pragma unroll
-  for (int t = 0; t < LMM_TILES; t++)
-#pragma unroll
-    for (int s = 0; s < LMM_KS; s++) {
-      const int k = k0 + 32 * s + 8 * g;
-      a[t][s] = k < n ? *reinterpret_cast<const lm_u32x4*>(wr[t] + k) : lm_u32x4{0u, 0u, 0u, 0u};
-    }
+// 16 bytes per lane from base + off to LDS at byte address lds + 16 lane.
+// (Written as asm because for the builtin the compiler orders every later
+// LDS read of the workgroup behind all such loads; the stage loop below
+// waits for exactly the loads that it needs.  M0, the LDS base, is written
+// by whatever uses it, right before its use.)
+__device__ __forceinline__ void lm_lds_load16(const void* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds), "v"(off), "s"(base)
+               : "memory");
+}
+// At most N of this wave's vector memory operations, and none of its LDS
+// operations, still outstanding.
+template <int N>
+__device__ __forceinline__ void lm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");
 }
 
-template <int NT>
-__device__ __forceinline__ void lm_mfma(const lm_u32x4 (&a)[LMM_TILES][LMM_KS],
-                                        const uint16_t* xs, lm_f32x4 (&acc)[LMM_TILES][NT],
-                                        uint32_t& bad, int m, int g) {
-#pragma unroll
-  for (int s = 0; s < LMM_KS; s++) {
-    lm_bf16x8 bx[3][NT];
-#pragma unroll
-    for (int p = 0; p < 3; p++)
-#pragma unroll
-      for (int j = 0; j < NT; j++)
-        bx[p][j] = *reinterpret_cast<const lm_bf16x8*>(
-            &xs[(p * 16 * NT + j * 16 + m) * LMM_RS + 32 * s + 8 * g]);
-#pragma unroll
-    for (int t = 0; t < LMM_TILES; t++) {
-      bad |= lm_nonfinite8(a[t][s]) ? 1u << t : 0u;
-      const lm_bf16x8 av = __builtin_bit_cast(lm_bf16x8, a[t][s]);
-#pragma unroll
-      for (int j = 0; j < NT; j++) {
-        // the largest part first: the small ones add to an accumulator of
-        // the product's own size
-        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bx[2][j], acc[t][j], 0, 0, 0);
-        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bx[1][j], acc[t][j], 0, 0, 0);
-        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bx[0][j], acc[t][j], 0, 0, 0);
-      }
-    }
-  }
-}
-
-// One chunk step of the pipeline: the next chunk's activations and weights
-// are loaded (activations first: converting them waits only for them) and
-// its activation parts stored in the other LDS buffer while this chunk's
-// MFMAs run; one barrier per chunk.
-template <int NT>
-__device__ __forceinline__ void lm_step(int k0, int n, const float* __restrict__ X, long ldx,
-                                        int nb, const uint16_t* const (&wr)[LMM_TILES],
-                                        const lm_u32x4 (&cur)[LMM_TILES][LMM_KS],
-                                        lm_u32x4 (&nxt)[LMM_TILES][LMM_KS], const uint16_t* xs_cur,
-                                        uint16_t* xs_nxt, lm_f32x4 (&acc)[LMM_TILES][NT],
-                                        uint32_t& bad, int m, int g) {
-  const bool more = k0 + LMM_KC < n;
-  LmX<NT> xr;
-  if (more) {
-    lm_x_load<NT>(xr, X, ldx, nb, n, k0 + LMM_KC);
-    lm_w_load(nxt, wr, n, k0 + LMM_KC, g);
-    lm_x_store<NT>(xr, xs_nxt);
-  }
-  lm_mfma<NT>(cur, xs_cur, acc, bad, m, g);
-  __syncthreads();
-}
-
-template <int NT, int MODE>
-__global__ __launch_bounds__(64 * LMM_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void k_lmhead_mfma(
-    const uint16_t* __restrict__ W, int V, int n, const float* __restrict__ X, long ldx, int nb,
-    float* __restrict__ logits, long ld, unsigned long long* __restrict__ keys, int kstride,
-    uint8_t* __restrict__ nan0) {
-  // the activation parts of two chunks (this one and the next): [2][3][16 NT][LMM_RS] bf16
-  __shared__ __align__(16) uint16_t xs[2][3 * 16 * NT * LMM_RS];
-  __shared__ unsigned long long best_sh[LMM_WAVES][16 * NT];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+template <int WR, int WC, int TR, int TC, int KS, int NS, int MODE>
+__global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2, 8))) void
+k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __restrict__ xp,
+              int ctt, int ncb, int nrt, const float* __restrict__ X, long ldx, int nb,
+              float* __restrict__ logits, long ld, unsigned long long* __restrict__ keys,
+              int kstride, uint8_t* __restrict__ nan0) {
+  constexpr int NW = WR * WC;                    // waves
+  constexpr int RF = WR * TR, CF = WC * TC;      // 16-row and 16-batch-row tiles
+  constexpr int WI = RF * KS, XF = CF * 3 * KS;  // 1 KiB loads of a stage: weights, parts
+  constexpr int WPW = WI / NW, XPW = (XF + NW - 1) / NW, PER = WPW + XPW;  // of a wave
+  constexpr int STG = (WI + XF) * LMX_FRAG;
+  static_assert(WI % NW == 0 && (KS == 1 || KS == 2) && (NS & 1) + NS > 1, "");
+  static_assert(TR % WC == 0 || WC % TR == 0, "");
+  static_assert((size_t)NS * STG * 2 >= NW * CF * 16 * 8, "the epilogue's keys reuse the ring");
+  __shared__ __align__(16) uint16_t sh[NS * STG];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, g = lane >> 4;
-  const int wrow0 = blockIdx.x * LMM_ROWS + w * LMM_TILES * 16;  // the wave's first row
-  lm_f32x4 acc[LMM_TILES][NT];
+  const int wr = w % WR, wc = w / WR;
+  // row tile rt and batch block cb: the batch blocks of a tile on one XCD
+  // (workgroups go to the eight XCDs in turn), one after the other
+  const int slot = blockIdx.x >> 3;
+  const int rt = (slot / ncb) * 8 + (blockIdx.x & 7), cb = slot % ncb;
+  if (rt >= nrt) return;
+  const int row0 = rt * RF * 16;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)sh;
+  const uint16_t* wbase = W + (size_t)row0 * n;
+  const int nst = (n + 32 * KS - 1) / (32 * KS);
+  // this wave's loads of W: row and 16-byte piece per lane.  Rows past V read
+  // row V - 1 (values unused); pieces past n read the row's last piece, which
+  // meets zero parts (and is non-finite only in a row flagged anyway).
+  uint32_t woff[WPW];
+  const int piece = KS == 1 ? g : (lane & 7) ^ (lane >> 3);
 #pragma unroll
-  for (int t = 0; t < LMM_TILES; t++)
-#pragma unroll
-    for (int j = 0; j < NT; j++) acc[t][j] = lm_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  // this lane's W rows (clamped into range: rows past V compute unused values)
-  const uint16_t* wr[LMM_TILES];
-#pragma unroll
-  for (int t = 0; t < LMM_TILES; t++) {
-    const int r = wrow0 + t * 16 + m;
-    wr[t] = W + (size_t)(r < V ? r : V - 1) * n;
+  for (int i = 0; i < WPW; i++) {
+    const int q = w * WPW + i;
+    const int r = KS == 1 ? q * 16 + m : q * 8 + (lane >> 3);
+    const int last = V - 1 - row0;
+    woff[i] = ((uint32_t)(r < last ? r : last) * (uint32_t)n + 8u * piece) * 2u;
   }
-  uint32_t bad = 0;  // bit t: this lane's row of tile t holds a non-finite weight
-  if (NT == 1) {
-    // two chunks' weights in registers: the next chunk's loads overlap this
-    // chunk's MFMAs
-    lm_u32x4 a0[LMM_TILES][LMM_KS], a1[LMM_TILES][LMM_KS];
-    {
-      LmX<NT> xr;
-      lm_x_load<NT>(xr, X, ldx, nb, n, 0);
-      lm_w_load(a0, wr, n, 0, g);
-      lm_x_store<NT>(xr, xs[0]);
+  const int klast = (nst - 1) * 32 * KS + 8 * piece;
+  const uint32_t wadj = klast < n ? 0u : (uint32_t)(klast - (n - 8)) * 2u;
+  const uint32_t xoff = (uint32_t)lane * 16u;
+  auto issue = [&](int c, int buf, int i) {  // load i of stage c into ring slot buf
+    const uint32_t l0 = lds0 + (uint32_t)buf * STG * 2;
+    if (i < WPW) {
+      lm_lds_load16(wbase + c * 32 * KS, woff[i] - (c == nst - 1 ? wadj : 0u),
+                    l0 + (w * WPW + i) * 1024);
+    } else {
+      int q = w * XPW + i - WPW;
+      if (XF % NW) q = q < XF ? q : XF - 1;  // (the same bytes to the same place again)
+      const int s = q / (CF * 3), e = q - s * CF * 3;
+      lm_lds_load16(xp + (((size_t)(c * KS + s) * ctt + cb * CF) * 3 + e) * LMX_FRAG, xoff,
+                    l0 + (WI + q) * 1024);
     }
-    __syncthreads();
-    for (int k0 = 0; k0 < n; k0 += 2 * LMM_KC) {
-      lm_step<NT>(k0, n, X, ldx, nb, wr, a0, a1, xs[0], xs[1], acc, bad, m, g);
-      if (k0 + LMM_KC >= n) break;
-      lm_step<NT>(k0 + LMM_KC, n, X, ldx, nb, wr, a1, a0, xs[1], xs[0], acc, bad, m, g);
-    }
-  } else {
-    // 32 batch rows: one chunk's weights in registers (two would spill at
-    // two workgroups per CU), every load of a chunk in flight before its
-    // MFMAs
-    for (int k0 = 0; k0 < n; k0 += LMM_KC) {
-      lm_u32x4 a[LMM_TILES][LMM_KS];
-      LmX<NT> xr;
-      lm_x_load<NT>(xr, X, ldx, nb, n, k0);
-      lm_w_load(a, wr, n, k0, g);
-      __syncthreads();  // the previous chunk's MFMAs are done with the LDS
-      lm_x_store<NT>(xr, xs[0]);
-      __syncthreads();
-      lm_mfma<NT>(a, xs[0], acc, bad, m, g);
-    }
-  }
-  // rows with a non-finite weight: fp32 fused multiply-adds over k (lanes),
-  // in every batch row, into the lanes that hold them (rare: a loop per row)
+  };
+  lm_f32x4 acc[TR][TC];
 #pragma unroll
-  for (int t = 0; t < LMM_TILES; t++) {
-    uint64_t rows_bad = __ballot((bad >> t) & 1u) ;
-    // lanes l, l + 16, l + 32, l + 48 share a row: fold the groups
-    const uint32_t rb = (uint32_t)(rows_bad | (rows_bad >> 16) | (rows_bad >> 32) | (rows_bad >> 48)) &
-                        0xffffu;
-    for (uint32_t mm = rb; mm; mm &= mm - 1u) {
-      const int r16 = (int)__builtin_ctz(mm);
-      const int row = wrow0 + t * 16 + r16;
-      if (row >= V) break;
-      const uint16_t* wrow = W + (size_t)row * n;
-      for (int b = 0; b < nb && b < 16 * NT; b++) {
-        float d = 0.0f;
-        for (int k = lane; k < n; k += 64)
-          d = __builtin_fmaf(lm_bf16_f(wrow[k]), X[(size_t)b * ldx + k], d);
-        d = pz_wave_sum(d);
-        if (g == (r16 >> 2) && m == (b & 15))
+  for (int t = 0; t < TR; t++)
 #pragma unroll
-          for (int j = 0; j < NT; j++)
-            if (j == (b >> 4))
+    for (int j = 0; j < TC; j++) acc[t][j] = lm_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // largest |weight| bits seen, two halves; the waves that share rows take
+  // their tiles in turn
+  lm_u16x2 wmax = {0, 0};
 #pragma unroll
-              for (int i = 0; i < 4; i++)
-                if (i == (r16 & 3)) acc[t][j][i] = d;
-      }
-    }
-  }
-  // epilogue: lane l holds batch row 16 j + l % 16, rows 4 (l / 16) + i of each tile
-  unsigned long long best[NT];
+  for (int i = 0; i < NS - 1; i++)
 #pragma unroll
-  for (int j = 0; j < NT; j++) best[j] = 0ull;
+    for (int q = 0; q < PER; q++) issue(i < nst ? i : nst - 1, i, q);
+  int buf = 0, nbuf = NS - 1;
+#pragma clang loop unroll(disable)
+  for (int c = 0; c < nst; c++) {
+    // stage c has arrived (the NS - 2 after it may be on their way), in every
+    // wave; and every wave is done reading the slot that is filled next
+    lm_wait<(NS - 2) * PER>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const uint16_t* sw = sh + buf * STG;
+    const uint16_t* sx = sw + WI * LMX_FRAG;
+    const int cn = c + NS - 1 < nst ? c + NS - 1 : nst - 1;  // (past the end: reloaded, unused)
 #pragma unroll
-  for (int t = 0; t < LMM_TILES; t++)
+    for (int s = 0; s < KS; s++) {
+      lm_bf16x8 a[TR], b[3][TC];
+      const uint16_t* sxs = sx + (s * CF + wc * TC) * 3 * LMX_FRAG + lane * 8;
 #pragma unroll
-    for (int j = 0; j < NT; j++) {
-      const int b = 16 * j + m;
+      for (int j = 0; j < TC; j++)
+        b[2][j] = *reinterpret_cast<const lm_bf16x8*>(sxs + (j * 3 + 2) * LMX_FRAG);
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int row = wrow0 + t * 16 + 4 * g + i;
-        const float v = acc[t][j][i];
-        if (row < V && b < nb) {
-          if (MODE == 0) {
-            logits[(size_t)b * ld + row] = v;
-          } else {
-            if (row == 0) nan0[b] = v != v ? 1 : 0;
-            if (!(v != v)) {
-              const unsigned long long kk = argmax_key(v, row);
-              best[j] = kk > best[j] ? kk : best[j];
+      for (int t = 0; t < TR; t++)
+        a[t] = *reinterpret_cast<const lm_bf16x8*>(
+            KS == 1 ? sw + (wr * TR + t) * LMX_FRAG + lane * 8
+                    : sw + (wr * TR + t) * 2 * LMX_FRAG + m * 64 + ((s * 4 + g) ^ (m & 7)) * 8);
+#pragma unroll
+      for (int p = 1; p >= 0; p--)
+#pragma unroll
+        for (int j = 0; j < TC; j++)
+          b[p][j] = *reinterpret_cast<const lm_bf16x8*>(sxs + (j * 3 + p) * LMX_FRAG);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int p = 2; p >= 0; p--)
+#pragma unroll
+        for (int j = 0; j < TC; j++)
+#pragma unroll
+          for (int t = 0; t < TR; t++) {
+            acc[t][j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[p][j], acc[t][j], 0, 0, 0);
+            // the next stage's loads, one every few MFMAs of the first k-step
+            constexpr int SP = 3 * TR * TC / PER >= 4 ? 4 : 3 * TR * TC / PER;
+            static_assert(SP >= 1, "");
+            const int q = ((2 - p) * TC + j) * TR + t;
+            if (s == 0 && q % SP == SP - 1 && q / SP < PER) {
+              issue(cn, nbuf, q / SP);
+              __builtin_amdgcn_sched_barrier(0);
             }
           }
+#pragma unroll
+      for (int t = 0; t < TR; t++)
+        if (WC == 1 || t % WC == wc % TR) {
+          const lm_u32x4 q = __builtin_bit_cast(lm_u32x4, a[t]);
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            wmax = __builtin_elementwise_max(wmax,
+                                             __builtin_bit_cast(lm_u16x2, q[e] & 0x7fff7fffu));
+        }
+    }
+    asm volatile("" ::: "memory");
+    buf = buf + 1 == NS ? 0 : buf + 1;
+    nbuf = nbuf + 1 == NS ? 0 : nbuf + 1;
+  }
+  lm_wait<0>();
+  __syncthreads();  // the ring is free
+  // an infinite or NaN weight anywhere in the workgroup's rows: those rows
+  // again with fp32 fused multiply-adds over k (lanes), into the lanes that
+  // hold them (rare: a loop per row)
+  int* flag = reinterpret_cast<int*>(sh);
+  if (tid == 0) *flag = 0;
+  __syncthreads();
+  if (__ballot(wmax[0] >= 0x7f80u || wmax[1] >= 0x7f80u) && lane == 0) atomicOr(flag, 1);
+  __syncthreads();
+  const bool fix = *flag != 0;
+  __syncthreads();
+  if (fix) {
+#pragma unroll
+    for (int t = 0; t < TR; t++)
+      for (int r16 = 0; r16 < 16; r16++) {
+        const int row = row0 + (wr * TR + t) * 16 + r16;
+        if (row >= V) break;
+        const uint16_t* wrow = W + (size_t)row * n;
+        bool nf = false;
+        for (int k = lane; k < n; k += 64) nf |= (wrow[k] & 0x7f80u) == 0x7f80u;
+        if (!__ballot(nf)) continue;
+        for (int bl = 0; bl < 16 * TC; bl++) {
+          const int b = (cb * CF + wc * TC) * 16 + bl;
+          if (b >= nb) break;
+          float d = 0.0f;
+          for (int k = lane; k < n; k += 64)
+            d = __builtin_fmaf(lm_bf16_f(wrow[k]), X[(size_t)b * ldx + k], d);
+          d = pz_wave_sum(d);
+          if (g == (r16 >> 2) && m == (bl & 15))
+#pragma unroll
+            for (int j = 0; j < TC; j++)
+              if (j == (bl >> 4))
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                  if (i == (r16 & 3)) acc[t][j][i] = d;
+        }
+      }
+  }
+  // epilogue: lane l holds batch row l % 16 of each tile, rows 4 (l / 16) + i
+  if (MODE == 0) {
+    const bool vec = (ld & 3) == 0 && ((uintptr_t)logits & 15) == 0;
+#pragma unroll
+    for (int j = 0; j < TC; j++) {
+      const int b = (cb * CF + wc * TC + j) * 16 + m;
+      if (b >= nb) continue;
+#pragma unroll
+      for (int t = 0; t < TR; t++) {
+        const int row = row0 + (wr * TR + t) * 16 + 4 * g;
+        float* o = logits + (size_t)b * ld + row;
+        if (vec && row + 3 < V) {
+          *reinterpret_cast<lm_f32x4*>(o) = acc[t][j];
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            if (row + i < V) o[i] = acc[t][j][i];
         }
       }
     }
-  if (MODE == 1) {
-    // the maximum key per batch row: over the four lane groups, then the waves
+  } else {
+    unsigned long long* best_sh = reinterpret_cast<unsigned long long*>(sh);  // [WR][CF * 16]
 #pragma unroll
-    for (int j = 0; j < NT; j++) {
+    for (int j = 0; j < TC; j++) {
+      const int bl = (wc * TC + j) * 16 + m, b = cb * CF * 16 + bl;
+      unsigned long long best = 0ull;
+#pragma unroll
+      for (int t = 0; t < TR; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int row = row0 + (wr * TR + t) * 16 + 4 * g + i;
+          const float v = acc[t][j][i];
+          if (row < V) {
+            if (row == 0 && b < nb) nan0[b] = v != v ? 1 : 0;
+            if (!(v != v)) {
+              const unsigned long long kk = argmax_key(v, row);
+              best = kk > best ? kk : best;
+            }
+          }
+        }
+      // the maximum over the four lane groups, then over the row waves
 #pragma unroll
       for (int off = 16; off < 64; off <<= 1) {
-        const unsigned long long o = __shfl_xor(best[j], off, 64);
-        best[j] = o > best[j] ? o : best[j];
+        const unsigned long long o = __shfl_xor(best, off, 64);
+        best = o > best ? o : best;
       }
-      if (g == 0) best_sh[w][16 * j + m] = best[j];
+      if (g == 0) best_sh[wr * CF * 16 + bl] = best;
     }
     __syncthreads();
-    if (tid < 16 * NT && tid < nb) {
-      unsigned long long mx = best_sh[0][tid];
-      for (int i = 1; i < LMM_WAVES; i++) mx = best_sh[i][tid] > mx ? best_sh[i][tid] : mx;
-      if (mx) atomicMax(&keys[(size_t)(blockIdx.x % LMM_SLOTS) * kstride + tid], mx);
+    for (int bl = tid; bl < CF * 16; bl += 64 * NW) {
+      const int b = cb * CF * 16 + bl;
+      if (b >= nb) break;
+      unsigned long long mx = best_sh[bl];
+#pragma unroll
+      for (int i = 1; i < WR; i++) {
+        const unsigned long long o = best_sh[i * CF * 16 + bl];
+        mx = o > mx ? o : mx;
+      }
+      if (mx) atomicMax(&keys[(size_t)(blockIdx.x % LMM_SLOTS) * kstride + b], mx);
     }
   }
 }
 
-template <int NT, int MODE>
+// One tile shape of the GEMM: its batch block, rows per workgroup, workgroups
+// per CU (LDS), k-steps per stage, and the time of one round of workgroups
+// on every CU at n = 2560 (us, measured at V = 128256).
+struct LmTile {
+  int cols, rows, per_cu;
+  float round_us;
+};
+constexpr LmTile LM_TILE_SHAPES[] = {
+    {256, 256, 1, 192.0f}, {128, 256, 1, 107.0f}, {64, 256, 1, 83.0f}, {32, 256, 1, 64.0f},
+    {32, 128, 2, 67.0f},   {16, 256, 1, 59.0f},   {16, 128, 2, 62.0f}};
+constexpr int LM_TILE_COUNT = sizeof(LM_TILE_SHAPES) / sizeof(LM_TILE_SHAPES[0]);
+
+// The shape with the least time for nb batch rows: rounds of workgroups times
+// a round's time.
+int lm_tile_for(int V, int nb, int most, int n_cu) {
+  int best = LM_TILE_COUNT - 1;
+  float best_us = __builtin_inff();
+  for (int i = 0; i < LM_TILE_COUNT; i++) {
+    const LmTile& t = LM_TILE_SHAPES[i];
+    if ((nb + t.cols - 1) / t.cols * t.cols > most) continue;  // parts past the workspace
+    const long wgs = (long)((V + t.rows - 1) / t.rows) * ((nb + t.cols - 1) / t.cols);
+    const long slots = (long)n_cu * t.per_cu;
+    const float us = (float)((wgs + slots - 1) / slots) * t.round_us;
+    if (us < best_us) {
+      best = i;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+template <int WR, int WC, int TR, int TC, int KS, int NS, int MODE>
 int launch_mfma(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* x, long ldx,
                 int nb, float* out, long ld, unsigned long long* keys, uint8_t* nan0) {
-  const int grid = (V + LMM_ROWS - 1) / LMM_ROWS;
-  hipLaunchKernelGGL((k_lmhead_mfma<NT, MODE>), dim3(grid), dim3(64 * LMM_WAVES), 0, s->stream,
-                     d_w, V, n, x, ldx, nb, out, ld, keys, s->max_batch, nan0);
+  constexpr int rows = WR * TR * 16, cols = WC * TC * 16;
+  const int ncb = (nb + cols - 1) / cols, nrt = (V + rows - 1) / rows, ctt = ncb * cols / 16;
+  const int ksteps = (n + 63) / 64 * 2;
+  hipLaunchKernelGGL(k_lmx_split, dim3(ksteps, ctt), dim3(64), 0, s->stream, x, ldx, nb, n, ctt,
+                     s->d_lmh_x);
+  PZ_HIP(s, hipGetLastError());
+  hipLaunchKernelGGL((k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE>),
+                     dim3((unsigned)((nrt + 7) / 8 * 8) * ncb), dim3(64 * WR * WC), 0, s->stream,
+                     d_w, V, n, s->d_lmh_x, ctt, ncb, nrt, x, ldx, nb, out, ld, keys,
+                     s->max_batch, nan0);
   PZ_HIP(s, hipGetLastError());
   return PZ_OK;
 }
@@ -478,6 +561,21 @@ int launch_tile(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* x
   return PZ_OK;
 }
 
+// The parts' workspace holds n weights of at least 16 batch rows: sized at
+// creation for PZ_LMX_ROWS rows of n = 8192 (or 16 rows of n = 131072); only
+// a longer row grows it.
+int lmx_reserve(pz_sampler* s, int n) {
+  const size_t need = (size_t)((n + 63) / 64) * 64 * 3 * 16;
+  if (need <= s->lmh_x_elems) return PZ_OK;
+  PZ_HIP(s, hipStreamSynchronize(s->stream));  // earlier calls may still read the old one
+  (void)hipFree(s->d_lmh_x);
+  s->d_lmh_x = nullptr;
+  s->lmh_x_elems = 0;
+  PZ_HIP(s, hipMalloc((void**)&s->d_lmh_x, need * sizeof(uint16_t)));
+  s->lmh_x_elems = need;
+  return PZ_OK;
+}
+
 // Batch tile: the largest of 8, 4, 2, 1 not above B whose x tile fits the
 // LDS budget (0: n too large even for one row).
 int tile_for(int B, int n) {
@@ -489,18 +587,34 @@ int tile_for(int B, int n) {
 template <int MODE>
 int run(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* d_x, int B, long ldx,
         float* d_logits, long ld) {
-  // batch 4 and up: the matrix cores, batch tiles of 32 (or 16), W 16-byte
-  // aligned with rows of a multiple of 8 weights
+  // batch 4 and up: the matrix cores, W 16-byte aligned with rows of a
+  // multiple of 8 weights; as many batch rows at a time as the parts'
+  // workspace holds, at most PZ_LMX_ROWS
   if (B >= 4 && n % 8 == 0 && ((uintptr_t)d_w & 15) == 0) {
-    for (int b0 = 0; b0 < B; b0 += 32) {
-      const int nb = B - b0 < 32 ? B - b0 : 32;
+    const int rc = lmx_reserve(s, n);
+    if (rc != PZ_OK) return rc;
+    const size_t fit = s->lmh_x_elems / ((size_t)((n + 63) / 64) * 64 * 3) / 16 * 16;
+    const int most = fit < (size_t)PZ_LMX_ROWS ? (int)fit : PZ_LMX_ROWS;
+    for (int b0 = 0; b0 < B; b0 += most) {
+      const int nb = B - b0 < most ? B - b0 : most;
       const float* x = d_x + (size_t)b0 * ldx;
       float* out = MODE == 0 ? d_logits + (size_t)b0 * ld : nullptr;
       unsigned long long* keys = s->d_lmh_keys + b0;
       uint8_t* nan0 = s->d_lmh_nan + b0;
-      const int rc = nb > 16 ? launch_mfma<2, MODE>(s, d_w, V, n, x, ldx, nb, out, ld, keys, nan0)
-                             : launch_mfma<1, MODE>(s, d_w, V, n, x, ldx, nb, out, ld, keys, nan0);
-      if (rc != PZ_OK) return rc;
+      int r;
+      switch (lm_tile_for(V, nb, most, s->n_cu)) {
+#define PZ_LM_CASE(I, ...) \
+  case I: r = launch_mfma<__VA_ARGS__, MODE>(s, d_w, V, n, x, ldx, nb, out, ld, keys, nan0); break
+        PZ_LM_CASE(0, 2, 4, 8, 4, 1, 2);
+        PZ_LM_CASE(1, 4, 2, 4, 4, 2, 2);
+        PZ_LM_CASE(2, 4, 2, 4, 2, 2, 2);
+        PZ_LM_CASE(3, 8, 1, 2, 2, 2, 3);
+        PZ_LM_CASE(4, 4, 1, 2, 2, 2, 2);
+        PZ_LM_CASE(5, 8, 1, 2, 1, 2, 4);
+        default: r = launch_mfma<4, 1, 2, 1, 2, 3, MODE>(s, d_w, V, n, x, ldx, nb, out, ld, keys, nan0);
+#undef PZ_LM_CASE
+      }
+      if (r != PZ_OK) return r;
     }
     return PZ_OK;
   }

@@ -113,6 +113,11 @@ extern "C" int pz_sampler_create(pz_sampler** out, int max_batch, int max_vocab,
       hipMalloc((void**)&s->d_lmh_keys, 16 * B * sizeof(unsigned long long)) != hipSuccess ||
       hipMalloc((void**)&s->d_lmh_nan, B) != hipSuccess)
     return bail(PZ_ENOMEM);
+  if (max_batch >= 4) {
+    s->lmh_x_elems = (size_t)PZ_LMX_ROWS * 8192 * 3;
+    if (hipMalloc((void**)&s->d_lmh_x, s->lmh_x_elems * sizeof(uint16_t)) != hipSuccess)
+      return bail(PZ_ENOMEM);
+  }
   // the fused LM head's argmax keys: 16 slots per row (zero between calls)
   if (hipMemset(s->d_lmh_keys, 0, 16 * B * sizeof(unsigned long long)) != hipSuccess)
     return bail(PZ_EDEVICE);
@@ -146,6 +151,7 @@ extern "C" void pz_sampler_destroy(pz_sampler* s) {
   (void)hipFree(s->d_eos);
   (void)hipFree(s->d_lmh_keys);
   (void)hipFree(s->d_lmh_nan);
+  (void)hipFree(s->d_lmh_x);
   (void)hipFree(s->d_scratch);
   (void)hipFree(s->d_split);
   (void)hipFree(s->spec_dev);

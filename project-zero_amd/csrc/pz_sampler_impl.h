@@ -9,6 +9,8 @@
 #include "pz_launch.h"
 #include "pz_params.h"
 
+constexpr int PZ_LMX_ROWS = 256;  // batch rows of one LM-head GEMM launch
+
 struct pz_sampler {
   int device = 0;
   int max_batch = 0, max_vocab = 0, max_hist = 0;
@@ -54,6 +56,10 @@ struct pz_sampler {
   // the NaN flag of logit 0 (max_batch each)
   unsigned long long* d_lmh_keys = nullptr;
   uint8_t* d_lmh_nan = nullptr;
+  // the LM head's activations as bf16 parts (samplers for batches of 4 or
+  // more): lmh_x_elems bf16, PZ_LMX_ROWS batch rows of n = 8192
+  uint16_t* d_lmh_x = nullptr;
+  size_t lmh_x_elems = 0;
 
   const float* call_u = nullptr;  // the synchronous call's host uniforms, during the call
 

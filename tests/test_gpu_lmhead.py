@@ -152,3 +152,50 @@ def test_fused_argmax_ties_and_nan(torch_cuda):
     assert np.isnan(logits[2, 0]) and ids[2] == 0
     assert ids[3] == 1
     check("ties", wb, x, logits, ids, gids, check_logits=False)
+
+
+# the matrix-core tile shapes: batch blocks of 16 .. 256 and their edges, two
+# chunks of 256, row tiles of 128 and 256 and their edges, k below one step,
+# off a step and off a stage
+@pytest.mark.parametrize("B,V,n", [
+    (4, 1, 8), (16, 129, 40), (17, 255, 96), (32, 4099, 1048), (33, 257, 72), (64, 512, 2560),
+    (65, 1000, 104), (128, 4099, 2056), (129, 300, 32), (256, 4099, 264), (257, 513, 160),
+    (530, 1025, 64), (20, 40000, 136), (100, 70001, 72), (200, 70001, 24), (90, 700, 24576)])
+def test_lm_head_matrix_core_tiles(torch_cuda, B, V, n):
+    """Every tile shape of the GEMM, unfused against float64 and fused against
+    the argmax of the unfused logits; row V // 2 holds an infinite weight (its
+    logits are +-inf by the sign of the activation it meets)."""
+    torch = torch_cuda
+    print(f"case lmhead tiles B={B} V={V} n={n}", flush=True)
+    rng = np.random.default_rng(B * 7 + n)
+    w = rng.standard_normal((V, n), dtype=np.float32) * 0.02
+    x = rng.standard_normal((B, n), dtype=np.float32)
+    r = V // 2
+    wb = bf16_bits(w)
+    finite = wb.copy()
+    wb[r, n - 1] = 0x7F80
+    finite[r] = 0
+    with pz.Sampler(B, max(V, 16)) as s:
+        logits, ids, gids = run(torch, wb, x, s)
+        # rows longer than their entries, off 16 bytes
+        ld, ldx = V + 3, n + 5
+        d_w = to_dev(torch, wb.view(np.int16))
+        d_x = torch.full((B, ldx), float("nan"), dtype=torch.float32, device="cuda")
+        d_x[:, :n] = to_dev(torch, x)
+        d_l = torch.full((B, ld), -7.0, dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        s.lm_head(d_w.data_ptr(), V, n, d_x, B, ldx, d_l, ld)
+        s.sync()
+        padded = d_l.cpu().numpy()
+    assert (logits[:, r] == np.copysign(np.inf, x[:, n - 1])).all()
+    assert (padded[:, :V].view(np.int32) == logits.view(np.int32)).all()
+    assert (padded[:, V:] == -7.0).all()
+    want = np.array([po.oracle().orc_argmax(
+        np.ascontiguousarray(q).ctypes.data_as(po._P), q.size) for q in logits], np.int32)
+    assert (ids == want).all() and (gids == ids).all()
+    logits[:, r] = 0.0
+    ex, bound = exact(finite, x)
+    err = np.abs(logits.astype(np.float64) - ex)
+    tol = n * 2.0 ** -24 * bound + 1e-30
+    print(f"B{B} V{V} n{n}: max |err| / bound = {float((err / tol).max()):.4f}", flush=True)
+    assert (err <= tol).all()
