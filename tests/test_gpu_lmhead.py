@@ -160,7 +160,7 @@ def test_fused_argmax_ties_and_nan(torch_cuda):
 @pytest.mark.parametrize("B,V,n", [
     (4, 1, 8), (16, 129, 40), (17, 255, 96), (32, 4099, 1048), (33, 257, 72), (64, 512, 2560),
     (65, 1000, 104), (128, 4099, 2056), (129, 300, 32), (256, 4099, 264), (257, 513, 160),
-    (530, 1025, 64), (20, 40000, 136), (100, 70001, 72), (200, 70001, 24), (90, 700, 24576)])
+    (530, 1025, 64), (9, 1025, 2048), (40, 800, 4096), (20, 40000, 136), (100, 70001, 72), (200, 70001, 24), (90, 700, 24576)])
 def test_lm_head_matrix_core_tiles(torch_cuda, B, V, n):
     """Every tile shape of the GEMM, unfused against float64 and fused against
     the argmax of the unfused logits; row V // 2 holds an infinite weight (its
