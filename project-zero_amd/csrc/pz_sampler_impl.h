@@ -141,6 +141,13 @@ int pz_dispatch_params(pz_sampler* s, const float* d_logits, int B, int V, long 
 int pz_launch_softmax_rows(pz_sampler* s, const float* d_in, long ld_in, float* d_out,
                            long ld_out, int B, int V, PzTemp T, const int32_t* d_len);
 
+// The same rows, each split over several workgroups in the workspace ws
+// (rows and ids within its size).  Returns 0, -1 (a launch failed) or -2 (the
+// workspace or the LDS does not hold the rows: nothing was launched).
+int pz_launch_softmax_split(pz_sampler* s, const PzSplitWs& ws, const float* d_in, long ld_in,
+                            float* d_out, long ld_out, int n_rows, int n, PzTemp T,
+                            const int32_t* d_len);
+
 // Launches the kernels for B rows whose kernel parameters are already in
 // s->res_params (n_params entries).  Used by the public entry points after
 // resolving pz_row_params, and by the reference-compatible calls, which set
