@@ -395,32 +395,46 @@ __device__ __forceinline__ int pz_rec_walk(PzAcc& st, const PzRec& R, int nseg, 
 // |d|: the fp32 product d*log2(e) carries an absolute error of about
 // |d| * 2^-23 in the exponent, plus v_exp_f32's own.  The bound used below,
 // (|d| + 2) * 2^-23, is checked on every fp32 d in [-104, 0] where expf(d)
-// is normal.  Only used where pz_inc_from_estimate can prove the rounding it
-// decides.
+// is normal.  Used for masses (predictions, histograms) that decide no
+// result.
 __device__ __forceinline__ float pz_fast_exp(float d) {
   return __builtin_amdgcn_exp2f(d * 1.44269504088896341f);
 }
 
-// Increment of a term at grid g from an estimate a of expf(d) (times a
-// factor rounded once more, for probabilities) when that settles the
-// rounding; otherwise sets *exact (the caller then evaluates the term
-// exactly).  The estimate's relative error is below (|d| + 3) * 2^-23; the
-// test uses twice that.  Grids below 2^-100 (only at the very start of a
-// row) always take the exact path, so estimates that underflow cannot
-// matter; so do terms of 2^20 grid steps or more, whose fraction fp32 no
-// longer resolves against the bound.
-// Branch-free (selects only): the value returned is meaningful only where
-// *exact is false.  a == 0 gives t = 0, fr = 0, no exact evaluation and 0.
-__device__ __forceinline__ uint32_t pz_inc_from_estimate(float a, float d, uint32_t g,
-                                                         bool* exact) {
-  const uint32_t gc = g < 50u ? 50u : g;
-  const float t = a * __uint_as_float((277u - gc) << 23);  // a / 2^(g - 150), exact
-  // the nearest integer and the distance to it: a fraction at least the
-  // margin away from one half rounds to that integer (round to nearest)
-  const float r = __builtin_rintf(t);
-  const float eps = (fabsf(d) + 3.0f) * 0x1p-22f;
-  *exact = (g < 50u) | (t >= 1048576.0f) | (0.5f - fabsf(t - r) <= t * eps + 0x1p-20f);
-  return (uint32_t)fminf(r, 1048576.0f);
+// A term on the grid g, estimated: t ~ expf(d) [* inv] / 2^(g - 150), as
+// exp2(d * log2(e) + k) [* mul] with the grid's exponent (and that of inv) in
+// k -- one fused multiply-add and one hardware exp2, no scaling after.
+// For t in [0.25, 2^20] (|the exponent| < 21) the relative error against the
+// exact term is at most, in units of 2^-24: the fma's rounding 2^-20 ln 2
+// (11.1), log2(e)'s rounding 0.22 |d|, v_exp_f32's ulp 2, the roundings of
+// expf, of p = e * inv and of the last product 1 each: 16.1 + 0.22 |d|, and
+// there |d| < 0.7 (170 - g).  eps is twice that; checked on every fp32 d in
+// [-104, 0] at every grid that puts t there, and for random inv.  Below 0.25
+// the term rounds to 0 whatever the error.
+struct PzIncScale {
+  float k, mul, eps;
+  bool low;  // a grid below 2^-100 (only at the very start of a row): no estimate
+};
+__device__ __forceinline__ PzIncScale pz_inc_scale(uint32_t g, float inv, bool as_p) {
+  PzIncScale s;
+  const uint32_t ib = __float_as_uint(inv);
+  const int e = as_p ? (int)(ib >> 23) - 127 : 0;  // (inv is normal: sums lie in [1, 2^18])
+  s.k = (float)(150 - (int)g + e);
+  s.mul = as_p ? __uint_as_float((ib & 0x7fffffu) | 0x3f800000u) : 1.0f;
+  s.eps = (32.0f + 0.31f * (float)(170 - (int)g)) * 0x1p-24f;
+  s.low = g < 50u;
+  return s;
+}
+__device__ __forceinline__ float pz_inc_est(float d, const PzIncScale& s, bool as_p) {
+  const float t =
+      __builtin_amdgcn_exp2f(__builtin_fmaf(d, 1.44269504088896341f, s.k));
+  return as_p ? t * s.mul : t;
+}
+// The estimate settles the increment (the nearest integer r): its fraction
+// stays at least the margin away from one half.  False for t >= 2^20 (whose
+// margin exceeds one half), an overflowed estimate and a NaN.
+__device__ __forceinline__ bool pz_inc_settled(float t, float r, const PzIncScale& s) {
+  return __builtin_fmaf(t, s.eps, fabsf(t - r)) < 0.5f - 0x1p-20f && !s.low;
 }
 
 // Terms of one row: e = expf(y - M) for y >= thr (0 otherwise), times inv
@@ -435,6 +449,10 @@ struct PzExpTerms {
   __device__ __forceinline__ int load(int e0, Raw& r) const { return R.load(e0, r); }
   __device__ __forceinline__ float exact_term(float y) const {
     const float e = y >= thr ? pz_expf_l(y - M, et) : 0.0f;
+    return as_p ? e * inv : e;
+  }
+  __device__ __forceinline__ float exact_term_inline(float y) const {
+    const float e = y >= thr ? pz_expf_tab(y - M, et) : 0.0f;
     return as_p ? e * inv : e;
   }
   __device__ __forceinline__ void prep(int e0, int n, Raw& r, float (&a)[4]) const {
@@ -467,20 +485,30 @@ struct PzExpTerms {
   // estimate settles is neither a tie nor big: both fail its test.)
   __device__ __forceinline__ void inc4(const Raw& y, const float (&a)[4], uint32_t g,
                                        uint32_t& s, bool& dirty) const {
+    (void)a;
+    const PzIncScale sc = pz_inc_scale(g, inv, as_p);
     uint32_t need = 0;
+    float sum = 0.0f;  // (four settled increments below 2^18: exact)
 #pragma unroll
     for (int c = 0; c < 4; c++) {  // (selects: no exec-mask branches per term)
-      bool ex;
-      const uint32_t i = pz_inc_from_estimate(a[c], y[c] - M, g, &ex);
+      const float t = pz_inc_est(y[c] - M, sc, as_p);
+      float r = __builtin_rintf(t);
+      bool ex = !pz_inc_settled(t, r, sc);
+      if (thr != -__builtin_inff()) {  // below the threshold: no term
+        const bool in = y[c] >= thr;
+        ex = ex && in;
+        r = in ? r : 0.0f;
+      }
       need |= (ex ? 1u : 0u) << c;
-      s += ex ? 0u : i;
+      sum += ex ? 0.0f : r;
     }
+    s += (uint32_t)sum;
     while (__ballot(need != 0u)) {
       if (need) {
         const int c = __builtin_ctz(need);
         need &= need - 1u;
         uint32_t cls;
-        s += pz_inc(exact_term(pz_sel4f(y[0], y[1], y[2], y[3], c)), g, &cls);
+        s += pz_inc(exact_term_inline(pz_sel4f(y[0], y[1], y[2], y[3], c)), g, &cls);
         dirty |= cls != PZ_INC_PLAIN;
       }
     }

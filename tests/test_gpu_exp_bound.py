@@ -27,6 +27,20 @@ def test_fast_exp_error_bound(torch_cuda):
     assert bad.value == 0
 
 
+@pytest.mark.parametrize("inv", [None, 1.0, 0.75, 0.1234567, 3.3e-5, 2.0 ** -18])
+def test_grid_estimate_within_half_its_margin(torch_cuda, inv):
+    """pz_inc_est, the estimate that settles most increments, against the exact
+    term at every fp32 exponent in [-104, 0] and every grid where it counts:
+    within half the margin the records leave (inv: the terms are expf * inv)."""
+    lib = ctypes.CDLL(LIB)
+    ratio, seen, lost = ctypes.c_float(), ctypes.c_uint(), ctypes.c_uint()
+    assert lib.pzcheck_inc_bound(ctypes.c_float(inv or 1.0), int(inv is not None),
+                                 ctypes.byref(ratio), ctypes.byref(seen), ctypes.byref(lost)) == 0
+    print(f"inv {inv}: max error / (margin / 2) = {ratio.value:.3f} (seen mod 2^32: {seen.value})")
+    assert 0.0 < ratio.value <= 1.0
+    assert lost.value == 0
+
+
 @pytest.mark.parametrize("lo,hi,stride", [
     (0x80000000, 0xC2D00000, 1),   # every fp32 in [-104, -0]: the sampler's exponents
     (0xC2D00000, 0xFF800000, 97),  # the underflowing tail down to -inf (sampled)
