@@ -540,7 +540,10 @@ int launch_spec(pz_sampler* s, SpecArgs& A) {
   // stat and records over the NR rows: about two rounds of workgroups (fewer,
   // larger slices leave a second round mostly empty; more add overhead)
   const PzSplitPlan pl = pz_split_plan(A.V, (A.NR + 1) / 2, A.ws.smax);
-  const PzSplitPlan pv = pz_split_plan(A.V, A.B, A.ws.smax);
+  // the draw's passes: one workgroup per CU, each sets up longer than it
+  // streams (32 sequences at 128256: estimate and records 12.1 + 18.8 us,
+  // with two per CU 15.4 + 24.9)
+  const PzSplitPlan pv = pz_split_plan(A.V, A.B, A.ws.smax, PZ_SP_TARGET_WG / 2);
   if (pl.nseg > A.ws.nsc) return -2;
   // two walking workgroups per CU fit when each takes at most half the LDS
   int nc = pz_sp_walk_nc(pl.nseg, (size_t)s->max_lds / 2 - fixed);
