@@ -9,7 +9,12 @@
 #include "pz_split.h"
 
 // Device scratch owned by a sampler (carved from one allocation).
-constexpr int PZ_FB_SLOTS = 32;        // rows the top-p fallback kernel sorts at once
+// Rows the top-p fallback kernel sorts at once: one per CU, as its LDS has it
+// (2 MiB of scratch each at 128256 ids, at most max_batch of them).  With 32,
+// 256 rows of 128256 ids at temperature 1, top-p 0.95 -- most of them wider
+// than the gather -- took 5282 us, where 256 slots take 972; 100 such rows of
+// 200000 ids 5562 and 1726.
+constexpr int PZ_FB_SLOTS = 256;
 constexpr int PZ_COUNTERS = 64;        // words of pz_scratch::counters
 constexpr int PZ_TOPP_MAX_V = 200000;  // top_p.c:27 (larger rows take argmax)
 constexpr int PZ_TOPP_CAPG = 12288;    // top-p candidates a row can gather for the LDS sort

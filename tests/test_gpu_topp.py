@@ -237,3 +237,14 @@ def test_cutoff_inside_the_first_segment_of_a_long_list(torch_cuda):
     check(torch_cuda, x, [pz.row_params(temperature=1.0, top_p=0.9)], u, label="long list")
     check(torch_cuda, x, [pz.row_params(temperature=1.0, top_p=0.9)], np.array([0.999, 0.0], np.float32),
           label="long list, u at the ends")
+
+
+@pytest.mark.parametrize("B", [70, 300])
+def test_many_rows_in_the_fallback(torch_cuda, B):
+    """Every row's nucleus is past the gather, in more rows than fit one round
+    of the fallback's sort slots (one per CU): each slot sorts several rows
+    one after the other."""
+    V = 15000
+    x = pz.synth_normal(B, V, 0.3, 0xFB)
+    u = pz.synth_draws(B, 0xFC)
+    check(torch_cuda, x, [pz.row_params(temperature=1.0, top_p=0.97)], u, label=f"fallback B={B}")
