@@ -5,7 +5,8 @@
 // qwen35_attention.c:156, qwen3moe_attention.c:136) all run
 // tn_softmax(att, valid_ctx) per head: softmax.c:4-23, i.e. the maximum by
 // strict '>' from x[0], e = expf(x - max), a sequential fp32 sum in index
-// order, x *= 1/sum.  Rows of up to 4096 scores take one wave each (four rows
+// order, x *= 1/sum.  Rows of up to ATTN_WAVE_SHORT scores, and many rows of up
+// to ATTN_WAVE_MAX, take one wave each (four rows
 // per 256-thread workgroup): the row sits in the wave's registers, 4
 // consecutive scores per lane per 256-score segment, so the maximum, the
 // exponentials, the exact sum and the write need no LDS beyond the exp
@@ -13,7 +14,7 @@
 // through the integer state -- a segment with at most one binade exit and
 // no tie before it in one step (pz_sp_fast) -- else, and for the first
 // segment, by its 256 real fp32 adds in order (the DPP chain, pz_sp_chain).  Rows of more than
-// ATTN_WAVE_SHORT scores (and up to ATTN_ROW_MAX) take one 1024-thread
+// that (and up to ATTN_ROW_MAX) take one 1024-thread
 // workgroup each instead (k_attn_row): its 16 waves estimate every 256-score
 // segment's mass, predict the binade the running sum sits in at each
 // segment, record the segments' integer increment sums there in LDS, and
@@ -40,18 +41,40 @@ constexpr int ATTN_WAVE_MAX = 16 * 256;     // longest row of the wave kernel
 // One 256-term segment added to the running sum st (the whole wave, lane l
 // holding terms 4l .. 4l+3): the one-step form when no tie or big term comes
 // before the term that leaves the binade, else the sequential chain of real
-// fp32 adds (always from a zero sum).  Out
-// of line so the unrolled segment loop holds one copy.
-__device__ __noinline__ PzAcc attn_seg_sum(PzAcc st, float a, float b, float c, float d) {
+// fp32 adds (always from a zero sum).  late: a segment far enough into the
+// row that two in three have no such term at all, tried first as the integer
+// sum of its increments at the state's grid (2048 ragged rows of up to 4096
+// scores: 35.9 -> 32.8 us).  Out of line so the unrolled segment loop holds
+// one copy.
+__device__ __noinline__ PzAcc attn_seg_sum(PzAcc st, float a, float b, float c, float d,
+                                           bool late) {
   const float v[4] = {a, b, c, d};
   if (st.n == 0u && st.g == 1u) {
     pz_sp_chain<PZ_STOP_NONE>(st, v, 0.0f);
   } else {
-    uint32_t P[4], Q[4], fP, fQ;
     const uint32_t g0 = st.g;
-    pz_sp_prefix4(v, g0, P, fP);
-    pz_sp_prefix4(v, g0 + 1u, Q, fQ);
-    if (!pz_sp_fast<PZ_STOP_NONE>(st, v, P, fP, Q, fQ, 0.0f)) pz_sp_chain<PZ_STOP_NONE>(st, v, 0.0f);
+    bool done = false;
+    if (late) {
+      uint32_t sum = 0;
+      bool odd = false;
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        uint32_t cls;
+        sum += pz_inc(v[k], g0, &cls);
+        odd |= cls != PZ_INC_PLAIN;
+      }
+      // (an increment is below 2^24, so 256 of them stay below 2^32)
+      const uint32_t total = pz_wave_sum_u32(sum);
+      done = !__ballot(odd) && total < (1u << 24) - st.n;
+      st.n += done ? total : 0u;
+    }
+    if (!done) {
+      uint32_t P[4], Q[4], fP, fQ;
+      pz_sp_prefix4(v, g0, P, fP);
+      pz_sp_prefix4(v, g0 + 1u, Q, fQ);
+      if (!pz_sp_fast<PZ_STOP_NONE>(st, v, P, fP, Q, fQ, 0.0f))
+        pz_sp_chain<PZ_STOP_NONE>(st, v, 0.0f);
+    }
   }
   pz_sp_uni(st);
   return st;
@@ -121,7 +144,7 @@ __global__ __launch_bounds__(64 * ATTN_WAVES) void k_attn_wave(const float* in, 
   const int nseg = (len + 255) >> 8;
 #pragma unroll
   for (int s = 0; s < NSEG; s++)
-    if (s < nseg) st = attn_seg_sum(st, v[s][0], v[s][1], v[s][2], v[s][3]);
+    if (s < nseg) st = attn_seg_sum(st, v[s][0], v[s][1], v[s][2], v[s][3], s >= 4);
   const float inv = 1.0f / pz_acc_value(st);  // softmax.c:19
 #pragma unroll
   for (int s = 0; s < NSEG; s++) {
@@ -445,7 +468,13 @@ extern "C" int pz_attn_softmax(pz_sampler* s, const float* d_in, long ld_in, flo
     if (rc == -3) return fail(s, PZ_ENOMEM, "attention softmax workspace");
     if (rc != -2) return fail(s, PZ_EDEVICE, "attention softmax launch failed");
   }
-  if (n > ATTN_WAVE_SHORT && n <= ATTN_ROW_MAX) {
+  // a workgroup per row runs one row per CU at a time, a wave per row all of
+  // them: beyond a round or two of workgroups the waves are quicker (us,
+  // workgroups / waves: n = 2048, 256 rows 14 / 19, 512 25 / 19, 2048 89 /
+  // 23; n = 4096, 512 rows 29 / 32, 1024 53 / 35, 2048 103 / 42)
+  const int cus = s->n_cu > 0 ? s->n_cu : 256;
+  const bool waves = n <= ATTN_WAVE_MAX && n_rows > (n <= 2048 ? cus : 2 * cus);
+  if (n > ATTN_WAVE_SHORT && n <= ATTN_ROW_MAX && !waves) {
     const int rc = launch_row(s, d_in, ld_in, d_out, ld_out, n_rows, n, d_len);
     if (rc == 0) return PZ_OK;
     if (rc != -2) return fail(s, PZ_EDEVICE, "attention softmax launch failed");

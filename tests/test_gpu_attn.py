@@ -123,3 +123,23 @@ def test_special_values(torch_cuda, n):
     x[11, 11] = 0.0
     print(f"case attn special n={n}", flush=True)
     run(torch_cuda, x, label=f"special{n}")
+
+
+@pytest.mark.parametrize("rows,n", [(256, 1025), (257, 1025), (300, 2048), (257, 2049),
+                                    (513, 2049), (515, 4095), (520, 4096), (600, 4097)])
+def test_many_rows(torch_cuda, rows, n):
+    """Around the row counts from which rows of up to 4096 scores take a wave
+    each instead of a workgroup, over ragged lengths, with rows whose sums
+    take every form of a segment (ties, exits, terms as large as the sum)."""
+    print(f"case attn many rows={rows} n={n}", flush=True)
+    rng = np.random.default_rng(rows + n)
+    x = scores(rows, n, 0xE0 + n, sigma=3.0)
+    x[1] = np.round(x[1])
+    x[2] *= 20.0
+    x[3] = 0.25
+    x[4, n // 2] = np.nan
+    x[5] = np.sort(x[5])        # the sum leaves a binade again and again
+    lens = rng.integers(1, n + 1, rows).astype(np.int32)
+    lens[:7] = [n, n, n, n, n, n, 0]
+    run(torch_cuda, x, lens=lens, label=f"many{rows}x{n}")
+    run(torch_cuda, x, label=f"manyfull{rows}x{n}")
