@@ -16,8 +16,10 @@
 //   * a workgroup of 4 waves owns 64 consecutive rows of W; the batch tile of
 //     x (BT rows x n fp32) is staged in LDS once per workgroup;
 //   * a wave takes 4 rows of W at a time; lane l covers elements
-//     512 c + 8 l .. +7 of every row (one 16-byte load per row per c), so a
-//     wave keeps 4 x n/512 loads in flight;
+//     512 c + 8 l .. +7 of every row (one 16-byte load per row per c), the
+//     next chunk's (or the next rows') loads on their way during a chunk's
+//     multiply-adds: 6.7 TB/s at 128256 x 2560, batch 1 (5.7 with the loads
+//     of a chunk waited for at once and cached);
 //   * each lane accumulates with fused multiply-adds in a fixed order (c,
 //     then the 8 elements), and a DPP tree sums the 64 lanes.
 // The order differs from the reference's AVX-512 accumulators, so logits
@@ -46,45 +48,73 @@ constexpr int LM_ROWS = 64;                     // rows per workgroup
 constexpr int LM_STEPS = LM_ROWS / (LM_WAVES * LM_RW);
 constexpr size_t LM_LDS_MAX = 96 * 1024;        // x tile budget
 
-__device__ __forceinline__ float bf16_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
-
 // The 8 weights of one 16-byte load (little-endian: element 2k is the low
 // half of word k).
-__device__ __forceinline__ void widen8(const uint4 q, float (&w)[8]) {
-  w[0] = __uint_as_float(q.x << 16);
-  w[1] = __uint_as_float(q.x & 0xffff0000u);
-  w[2] = __uint_as_float(q.y << 16);
-  w[3] = __uint_as_float(q.y & 0xffff0000u);
-  w[4] = __uint_as_float(q.z << 16);
-  w[5] = __uint_as_float(q.z & 0xffff0000u);
-  w[6] = __uint_as_float(q.w << 16);
-  w[7] = __uint_as_float(q.w & 0xffff0000u);
+typedef uint32_t lm_u32x4 __attribute__((ext_vector_type(4)));
+typedef float lm_f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void widen8(const lm_u32x4 q, float (&w)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    w[2 * i] = __uint_as_float(q[i] << 16);
+    w[2 * i + 1] = __uint_as_float(q[i] & 0xffff0000u);
+  }
 }
 
 __device__ __forceinline__ uint64_t argmax_key(float v, int id) {
   return ((uint64_t)pz_key(v) << 32) | (uint64_t)(0xffffffffu - (uint32_t)id);
 }
 
+// Weights the Infinity Cache (256 MB) cannot hold from one call to the next
+// are loaded non-temporally: 128256 x 2560 at batch 1 114 -> 98 us, at 8
+// (matrix cores) 116 -> 107; 50257 x 1024, which it can hold, 18.2 -> 19.5.
+bool lm_once(int V, int n) { return (size_t)V * n * 2 > ((size_t)256 << 20); }
+
 // MODE 0: write logits.  MODE 1: argmax keys.  VEC: n % 8 == 0 and W 16-byte
 // aligned (one 16-byte load per 8 weights), else element loads.
-template <int BT, int MODE, bool VEC>
+template <int BT, int MODE, bool VEC, bool NT>
 __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
     const uint16_t* __restrict__ W, int V, int n, const float* __restrict__ X, long ldx, int nb,
     float* __restrict__ logits, long ld, unsigned long long* __restrict__ keys,
     uint8_t* __restrict__ nan0) {
-  extern __shared__ __align__(16) float xs[];  // [BT][n]
+  extern __shared__ __align__(16) float xs[];  // [BT][n rounded up to 512]
   __shared__ unsigned long long best_sh[LM_WAVES][BT];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nchunk = (n + 511) >> 9;
+  // the wave's weights, one chunk of its 4 rows ahead of the multiply-adds
+  // (the first before the activations are staged)
+  const int wrow0 = blockIdx.x * LM_ROWS + w * LM_RW;
+  lm_u32x4 q[LM_RW];
+  auto fetch = [&](int r0, int c) {
+    const int k = c * 512 + lane * 8;
+#pragma unroll
+    for (int r = 0; r < LM_RW; r++) {
+      const int row = r0 + r < V ? r0 + r : V - 1;  // rows past V: a valid row, result unused
+      const uint16_t* wr = W + (size_t)row * n;
+      q[r] = lm_u32x4{0u, 0u, 0u, 0u};
+      if (VEC) {
+        const lm_u32x4* p = reinterpret_cast<const lm_u32x4*>(wr + k);
+        if (k < n) q[r] = NT ? __builtin_nontemporal_load(p) : *p;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const uint32_t h = k + e < n ? wr[k + e] : 0u;
+          q[r][e >> 1] |= h << (16 * (e & 1));
+        }
+      }
+    }
+  };
+  if (wrow0 < V) fetch(wrow0, 0);
+  const int ns = nchunk * 512;  // a staged row: zeros past n
   for (int b = 0; b < BT; b++)
-    for (int j = tid; j < n; j += 64 * LM_WAVES)
-      xs[b * n + j] = b < nb ? X[(size_t)b * ldx + j] : 0.0f;
+    for (int j = tid; j < ns; j += 64 * LM_WAVES)
+      xs[b * ns + j] = b < nb && j < n ? X[(size_t)b * ldx + j] : 0.0f;
   __syncthreads();
   unsigned long long best[BT];
 #pragma unroll
   for (int b = 0; b < BT; b++) best[b] = 0ull;
-  const int nchunk = (n + 511) >> 9;
   for (int step = 0; step < LM_STEPS; step++) {
-    const int r0 = blockIdx.x * LM_ROWS + (step * LM_WAVES + w) * LM_RW;
+    const int r0 = wrow0 + step * LM_WAVES * LM_RW;
     if (r0 >= V) break;  // whole wave
     float acc[LM_RW][BT];
 #pragma unroll
@@ -95,23 +125,18 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
       const int k = c * 512 + lane * 8;
       float wv[LM_RW][8];
 #pragma unroll
-      for (int r = 0; r < LM_RW; r++) {
-        const int row = r0 + r < V ? r0 + r : V - 1;  // rows past V: a valid row, result unused
-        const uint16_t* wr = W + (size_t)row * n;
-        if (VEC) {
-          uint4 q = make_uint4(0u, 0u, 0u, 0u);
-          if (k < n) q = *reinterpret_cast<const uint4*>(wr + k);
-          widen8(q, wv[r]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; e++) wv[r][e] = k + e < n ? bf16_to_f32(wr[k + e]) : 0.0f;
-        }
+      for (int r = 0; r < LM_RW; r++) widen8(q[r], wv[r]);
+      {
+        // the next chunk, or the next rows' first
+        const bool more = c + 1 < nchunk;
+        const int rn = more ? r0 : r0 + LM_WAVES * LM_RW;
+        if (more || (step + 1 < LM_STEPS && rn < V)) fetch(rn, more ? c + 1 : 0);
       }
 #pragma unroll
       for (int b = 0; b < BT; b++) {
-        float xv[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) xv[e] = k + e < n ? xs[b * n + k + e] : 0.0f;
+        const lm_f32x4 x0 = *reinterpret_cast<const lm_f32x4*>(&xs[b * ns + k]);
+        const lm_f32x4 x1 = *reinterpret_cast<const lm_f32x4*>(&xs[b * ns + k + 4]);
+        const float xv[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
 #pragma unroll
         for (int r = 0; r < LM_RW; r++)
 #pragma unroll
@@ -178,11 +203,14 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
 //     (global_load_lds_dwordx4) NS - 1 stages ahead, one barrier per stage,
 //     the loads spread between the stage's MFMAs.
 //   * KS = 2: one load instruction takes 8 rows x 128 bytes of W, whole
-//     cache lines (64-byte pieces, KS = 1, reach 4.0 TB/s at 16 batch rows
-//     where KS = 2 reaches 5.4); the 16-byte pieces of a row are rotated by
+//     cache lines (64-byte pieces, KS = 1, reach 4.2 TB/s at 16 batch rows
+//     where KS = 2 reaches 5.6); the 16-byte pieces of a row are rotated by
 //     XOR with the row in the source address so that the fragment reads do
 //     not meet in the banks.  The 256 x 256 tile's stage only fits with
 //     KS = 1; it is bound by the matrix cores, not by that.
+//   * 128256 x 2560: 16 batch rows 112 us, 32 124, 64 167, 128 237, 256 405
+//     (one launch per 32 rows that split the activations in every workgroup
+//     took 143, 152, 301, 601 and 1203).
 //   * Bounds: above about 64 batch rows the three parts' 6 V n B operations
 //     (1.3 PFLOP/s at 256 rows, against 1.65 for a large library bf16 product
 //     on the same card), below that one read of W.
@@ -190,8 +218,6 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
 // so its L2 serves W to all but the first.
 // MODE 1 (argmax keys) as in k_lmhead.
 typedef __bf16 lm_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float lm_f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t lm_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t lm_u16x2 __attribute__((ext_vector_type(2)));
 constexpr int LMX_FRAG = 512;  // bf16 of one fragment (16 x 32)
 
@@ -236,11 +262,18 @@ __global__ __launch_bounds__(64) void k_lmx_split(const float* __restrict__ X, l
 // LDS read of the workgroup behind all such loads; the stage loop below
 // waits for exactly the loads that it needs.  M0, the LDS base, is written
 // by whatever uses it, right before its use.)
+template <bool NT>
 __device__ __forceinline__ void lm_lds_load16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(lds), "v"(off), "s"(base)
-               : "memory");
+  if (NT)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                 :
+                 : "s"(lds), "v"(off), "s"(base)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds), "v"(off), "s"(base)
+                 : "memory");
 }
 // At most N of this wave's vector memory operations, and none of its LDS
 // operations, still outstanding.
@@ -249,7 +282,7 @@ __device__ __forceinline__ void lm_wait() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");
 }
 
-template <int WR, int WC, int TR, int TC, int KS, int NS, int MODE>
+template <int WR, int WC, int TR, int TC, int KS, int NS, int MODE, bool NT>
 __global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __restrict__ xp,
               int ctt, int ncb, int nrt, const float* __restrict__ X, long ldx, int nb,
@@ -301,13 +334,13 @@ k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __re
     const int c = cc + rot < nst ? cc + rot : cc + rot - nst;
     const uint32_t l0 = lds0 + (uint32_t)buf * STG * 2;
     if (i < WPW) {
-      lm_lds_load16(wbase + c * 32 * KS, woff[i] - (c == nst - 1 ? wadj : 0u),
-                    l0 + (w * WPW + i) * 1024);
+      const uint32_t off = woff[i] - (c == nst - 1 ? wadj : 0u), to = l0 + (w * WPW + i) * 1024;
+      lm_lds_load16<NT>(wbase + c * 32 * KS, off, to);
     } else {
       int q = w * XPW + i - WPW;
       if (XF % NW) q = q < XF ? q : XF - 1;  // (the same bytes to the same place again)
       const int s = q / (CF * 3), e = q - s * CF * 3;
-      lm_lds_load16(xp + (((size_t)(c * KS + s) * ctt + cb * CF) * 3 + e) * LMX_FRAG, xoff,
+      lm_lds_load16<false>(xp + (((size_t)(c * KS + s) * ctt + cb * CF) * 3 + e) * LMX_FRAG, xoff,
                     l0 + (WI + q) * 1024);
     }
   };
@@ -525,8 +558,11 @@ int launch_mfma(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* x
   hipLaunchKernelGGL(k_lmx_split, dim3(ksteps, ctt), dim3(64), 0, s->stream, x, ldx, nb, n, ctt,
                      s->d_lmh_x);
   PZ_HIP(s, hipGetLastError());
-  hipLaunchKernelGGL((k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE>),
-                     dim3((unsigned)((nrt + 7) / 8 * 8) * ncb), dim3(64 * WR * WC), 0, s->stream,
+  // (the 256-row tile is bound by the matrix cores: plain loads)
+  auto k = lm_once(V, n) && cols <= 128
+               ? k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE, (cols <= 128)>
+               : k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE, false>;
+  hipLaunchKernelGGL(k, dim3((unsigned)((nrt + 7) / 8 * 8) * ncb), dim3(64 * WR * WC), 0, s->stream,
                      d_w, V, n, s->d_lmh_x, ctt, ncb, nrt, x, ldx, nb, out, ld, keys,
                      s->max_batch, nan0);
   PZ_HIP(s, hipGetLastError());
@@ -552,12 +588,16 @@ __global__ void k_lmhead_finish(int B, unsigned long long* keys, int kstride, co
   keys[b] = 0ull;
 }
 
+// LDS of the vector kernel: bt activation rows of n rounded up to 512.
+size_t lm_x_bytes(int bt, int n) { return (size_t)bt * ((n + 511) / 512) * 512 * sizeof(float); }
+
 template <int BT, int MODE>
 int launch_tile(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* x, long ldx, int nb,
                 float* out, long ld, unsigned long long* keys, uint8_t* nan0) {
   const bool vec = n % 8 == 0 && ((uintptr_t)d_w & 15) == 0;
-  auto k = vec ? k_lmhead<BT, MODE, true> : k_lmhead<BT, MODE, false>;
-  const size_t lds = (size_t)BT * n * sizeof(float);
+  auto k = !vec ? k_lmhead<BT, MODE, false, false>
+                : (lm_once(V, n) ? k_lmhead<BT, MODE, true, true> : k_lmhead<BT, MODE, true, false>);
+  const size_t lds = lm_x_bytes(BT, n);
   if (lds > 65536)
     PZ_HIP(s, hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)lds));
@@ -583,12 +623,13 @@ int lmx_reserve(pz_sampler* s, int n) {
   return PZ_OK;
 }
 
-// Batch tile: the largest of 8, 4, 2, 1 not above B whose x tile fits the
-// LDS budget (0: n too large even for one row).
+// Batch tile: the smallest of 1, 2, 4, 8 that holds B rows (so three rows are
+// one read of W, not two), or the largest whose x tile fits the LDS budget
+// (0: n too large even for one row).
 int tile_for(int B, int n) {
-  for (int bt = 8; bt >= 1; bt >>= 1)
-    if (bt <= B && (size_t)bt * n * sizeof(float) <= LM_LDS_MAX) return bt;
-  return (size_t)n * sizeof(float) <= LM_LDS_MAX ? 1 : 0;
+  int bt = B <= 1 ? 1 : (B <= 2 ? 2 : (B <= 4 ? 4 : 8));
+  while (bt >= 1 && lm_x_bytes(bt, n) > LM_LDS_MAX) bt >>= 1;
+  return bt;
 }
 
 template <int MODE>
