@@ -81,7 +81,8 @@ __device__ __noinline__ PzAcc attn_seg_sum(PzAcc st, float a, float b, float c, 
 }
 
 // Row of NSEG segments (256 scores each, lane l: scores 256s + 4l .. +3).
-template <int NSEG, bool VEC_IN, bool VEC_OUT>
+// VI, VO: 16-byte loads and stores, at any address (pz_f4u).
+template <int NSEG, bool VI, bool VO>
 __global__ __launch_bounds__(64 * ATTN_WAVES) void k_attn_wave(const float* in, long ld_in,
                                                               float* out, long ld_out,
                                                               int n_rows, int n,
@@ -103,8 +104,8 @@ __global__ __launch_bounds__(64 * ATTN_WAVES) void k_attn_wave(const float* in, 
 #pragma unroll
   for (int s = 0; s < NSEG; s++) {
     const int i0 = s * 256 + 4 * lane;
-    if (VEC_IN && i0 + 3 < len) {
-      const pz_f4 q = *reinterpret_cast<const pz_f4*>(x + i0);
+    if (VI && i0 + 3 < len) {
+      const pz_f4u q = *reinterpret_cast<const pz_f4u*>(x + i0);
       v[s][0] = q.x;
       v[s][1] = q.y;
       v[s][2] = q.z;
@@ -149,13 +150,13 @@ __global__ __launch_bounds__(64 * ATTN_WAVES) void k_attn_wave(const float* in, 
 #pragma unroll
   for (int s = 0; s < NSEG; s++) {
     const int i0 = s * 256 + 4 * lane;
-    if (VEC_OUT && i0 + 3 < len) {
-      pz_f4 q;
+    if (VO && i0 + 3 < len) {
+      pz_f4u q;
       q.x = v[s][0] * inv;
       q.y = v[s][1] * inv;
       q.z = v[s][2] * inv;
       q.w = v[s][3] * inv;
-      *reinterpret_cast<pz_f4*>(o + i0) = q;
+      *reinterpret_cast<pz_f4u*>(o + i0) = q;
     } else {
 #pragma unroll
       for (int c = 0; c < 4; c++)
@@ -167,10 +168,15 @@ __global__ __launch_bounds__(64 * ATTN_WAVES) void k_attn_wave(const float* in, 
 template <int NSEG>
 int launch_wave(pz_sampler* s, const float* d_in, long ld_in, float* d_out, long ld_out,
                 int n_rows, int n, const int32_t* d_len) {
+  // rows off 16 bytes take 16-byte accesses too, but for the shortest, whose
+  // few lanes past them would wait twice (1024 rows of up to 101 scores 5.3
+  // us, 5.6 with them)
   const bool vi = (ld_in % 4 == 0) && (((uintptr_t)d_in & 15) == 0);
   const bool vo = (ld_out % 4 == 0) && (((uintptr_t)d_out & 15) == 0);
-  auto k = vi ? (vo ? k_attn_wave<NSEG, true, true> : k_attn_wave<NSEG, true, false>)
-              : (vo ? k_attn_wave<NSEG, false, true> : k_attn_wave<NSEG, false, false>);
+  const bool i = vi || NSEG > 2, o = vo || NSEG > 2;
+  auto k = i ? (o ? k_attn_wave<NSEG, true, true> : k_attn_wave<NSEG, true, (NSEG > 2)>)
+             : (o ? k_attn_wave<NSEG, (NSEG > 2), true>
+                  : k_attn_wave<NSEG, (NSEG > 2), (NSEG > 2)>);
   const int blocks = (n_rows + ATTN_WAVES - 1) / ATTN_WAVES;
   hipLaunchKernelGGL(k, dim3(blocks), dim3(64 * ATTN_WAVES), 0, s->stream, d_in, ld_in, d_out,
                      ld_out, n_rows, n, d_len);
@@ -208,7 +214,7 @@ struct AttnShared {
 // NSW: segments per wave (rows of up to 16 NSW segments); each wave holds
 // its segments' scores (segments w, w + 16, ...) in registers through the
 // records, and reads them once more for the probabilities.
-template <int NSW, bool VEC_IN, bool VEC_OUT>
+template <int NSW, bool VEC_IN>
 __global__ __launch_bounds__(AR_BLOCK) void k_attn_row(const float* in, long ld_in, float* out,
                                                       long ld_out, int n_rows, int n,
                                                       const int32_t* lens, int nc) {
@@ -379,13 +385,13 @@ __global__ __launch_bounds__(AR_BLOCK) void k_attn_row(const float* in, long ld_
 #pragma unroll
     for (int c = 0; c < 4; c++) v[c] = c < cnt[j] ? X.exact_term(y[j][c]) * inv : 0.0f;
     const int i0 = k * PZ_SP_SEG + 4 * lane;
-    if (VEC_OUT && i0 + 3 < len) {
-      pz_f4 q;
+    if (i0 + 3 < len) {
+      pz_f4u q;
       q.x = v[0];
       q.y = v[1];
       q.z = v[2];
       q.w = v[3];
-      *reinterpret_cast<pz_f4*>(o + i0) = q;
+      *reinterpret_cast<pz_f4u*>(o + i0) = q;
     } else {
 #pragma unroll
       for (int c = 0; c < 4; c++)
@@ -398,9 +404,7 @@ template <int NSW>
 int launch_row_t(pz_sampler* s, const float* d_in, long ld_in, float* d_out, long ld_out,
                  int n_rows, int n, const int32_t* d_len, int nc, size_t lds) {
   const bool vi = (ld_in % 4 == 0) && (((uintptr_t)d_in & 15) == 0);
-  const bool vo = (ld_out % 4 == 0) && (((uintptr_t)d_out & 15) == 0);
-  auto k = vi ? (vo ? k_attn_row<NSW, true, true> : k_attn_row<NSW, true, false>)
-              : (vo ? k_attn_row<NSW, false, true> : k_attn_row<NSW, false, false>);
+  auto k = vi ? k_attn_row<NSW, true> : k_attn_row<NSW, false>;
   if (lds > 65536 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)lds) != hipSuccess)
     return -1;

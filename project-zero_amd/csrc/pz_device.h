@@ -12,6 +12,9 @@
 
 // Native 128-bit vector (HIP's float4 is a struct; the builtins want this).
 typedef float pz_f4 __attribute__((ext_vector_type(4)));
+// Four floats at any float's address: still one 16-byte access (rows of an
+// odd stride, such as contiguous rows of 50257 ids).
+typedef float pz_f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // ---------------------------------------------------------------------------
 // Row addressing.  A launch either covers rows 0..n-1 or the rows named in a

@@ -13,13 +13,15 @@
 // groups tid, tid+BLOCK, ... in ascending id order.  Two register sets of U
 // float4 alternate: one set's loads are in flight while the other is
 // compared, and the first set is issued before the history bitmap is built.
+#include <type_traits>
+
 #include "pz_device.h"
 #include "pz_launch.h"
 
 namespace {
 
-template <int BLOCK, int U>
-__device__ __forceinline__ void gr_load(const pz_f4* x4, int n4, int base, pz_f4 (&v)[U]) {
+template <int BLOCK, int U, class F4>
+__device__ __forceinline__ void gr_load(const F4* x4, int n4, int base, pz_f4 (&v)[U]) {
 #pragma unroll
   for (int u = 0; u < U; u++) {
     const int i4 = base + u * BLOCK + (int)threadIdx.x;
@@ -93,9 +95,9 @@ __device__ __forceinline__ void gr_group(const PzPenalty& P, const pz_row_params
 // One exit only (the loop condition): a break in the middle of the loop body
 // makes the compiler merge paths on which the other set's loads are still
 // in flight, and it then drains every load at the loop head.
-template <int BLOCK, int U, bool TEMPER, bool PEN>
+template <int BLOCK, int U, bool TEMPER, bool PEN, class F4>
 __device__ __forceinline__ void gr_stream(const PzPenalty& P, const pz_row_params_dev& prm,
-                                          int lo, const pz_f4* x4, int n4, pz_f4 (&a)[U],
+                                          int lo, const F4* x4, int n4, pz_f4 (&a)[U],
                                           pz_f4 (&b)[U], GrBest& B) {
   constexpr int STEP = BLOCK * U;
   const int ng = (n4 + STEP - 1) / STEP;
@@ -117,7 +119,17 @@ __device__ __forceinline__ void gr_stream(const PzPenalty& P, const pz_row_param
 // guard, which take the argmax of the tempered row (top_p.c:33-34, after
 // apply_temperature).  PEN: some row of the launch has an active penalty;
 // every row then builds the bitmap (all zero where the row has none).
-template <int BLOCK, int U, bool VEC, bool TEMPER, bool PEN>
+// VEC: 2 rows start 16-byte aligned, 1 at any address (pz_f4u), 0 fewer than
+// four ids.
+template <int VEC>
+struct GrF4 {
+  typedef pz_f4 type;
+};
+template <>
+struct GrF4<1> {
+  typedef pz_f4u type;
+};
+template <int BLOCK, int U, int VEC, bool TEMPER, bool PEN>
 __global__ __launch_bounds__(BLOCK) void k_greedy(
     const float* __restrict__ logits, long ld, int V,
     const int32_t* __restrict__ rows, const pz_row_params_dev* __restrict__ params,
@@ -132,7 +144,8 @@ __global__ __launch_bounds__(BLOCK) void k_greedy(
   const float* x = logits + (long)row * ld;
   const int32_t* hrow = hist ? hist + (long)row * H : nullptr;
   const int tid = threadIdx.x;
-  const pz_f4* x4 = reinterpret_cast<const pz_f4*>(x);
+  typedef typename GrF4<VEC>::type F4;
+  const F4* x4 = reinterpret_cast<const F4*>(x);
   const int n4 = VEC ? V >> 2 : 0;  // VEC launches have V >= 4, so n4 >= 1
 
   // Prologue ordered for the in-order load counter: the history id of one
@@ -227,7 +240,7 @@ __global__ __launch_bounds__(BLOCK) void k_greedy(
 // value's key) when y[0] is NaN, which returns id 0.  The workgroup that
 // arrives last takes the largest word (pz_sp_post_last).  words: the row's
 // meeting words (zero between launches); arrive: zero between launches.
-template <int BLOCK, int U, bool TEMPER, bool PEN>
+template <int BLOCK, int U, int VEC, bool TEMPER, bool PEN>
 __global__ __launch_bounds__(BLOCK) void k_greedy_split(
     const float* __restrict__ logits, long ld, int V, int chunk,
     const int32_t* __restrict__ rows, const pz_row_params_dev* __restrict__ params,
@@ -246,7 +259,8 @@ __global__ __launch_bounds__(BLOCK) void k_greedy_split(
   const float* x = logits + (long)row * ld;
   const int32_t* hrow = hist ? hist + (long)row * H : nullptr;
   const int tid = threadIdx.x;
-  const pz_f4* x4 = reinterpret_cast<const pz_f4*>(x + lo);
+  typedef typename GrF4<VEC>::type F4;
+  const F4* x4 = reinterpret_cast<const F4*>(x + lo);
   const int n4 = (hi - lo) >> 2;  // 0 only for a last range of 1-3 ids
 
   int hid0 = -1;
@@ -386,15 +400,22 @@ template <bool TEMPER>
 static int launch_argmax(const pz_launch& L, int n_rows, const int32_t* d_rows) {
   if (n_rows <= 0) return 0;
   constexpr size_t kStatic = 2 * (GREEDY_BLOCK / PZ_WAVE) * 4;
-  const bool vec = (L.ld % 4 == 0) && (((uintptr_t)L.logits & 15) == 0) && L.V >= 4;
+  // 16-byte loads at any row address: contiguous rows of an odd number of ids
+  // stream and split over workgroups as aligned ones do (128257 ids, B = 1
+  // 66 -> 13 us, B = 64 109 -> 18, B = 256 151 -> 32 a call; one element per
+  // load and one workgroup per row before)
+  const int vec = L.V < 4 ? 0 : (L.ld % 4 == 0) && (((uintptr_t)L.logits & 15) == 0) ? 2 : 1;
   int chunk = 0;
   const int S = vec && L.ws.meet && L.ws.arrive ? greedy_split(L.V, n_rows, &chunk) : 1;
   if (S > 1 && S <= 2 * L.ws.smax) {
     const size_t lds = L.pen_any ? pz_penalty_lds_bytes(chunk, L.hcap) : 0;
     constexpr size_t kStaticS = 2 * (GREEDY_SPLIT_BLOCK / PZ_WAVE) * 4;
     if (lds + kStaticS > (size_t)L.max_lds) return -2;
-    auto k = L.pen_any ? k_greedy_split<GREEDY_SPLIT_BLOCK, GREEDY_SPLIT_U, TEMPER, true>
-                       : k_greedy_split<GREEDY_SPLIT_BLOCK, GREEDY_SPLIT_U, TEMPER, false>;
+    auto k = vec == 2
+                 ? (L.pen_any ? k_greedy_split<GREEDY_SPLIT_BLOCK, GREEDY_SPLIT_U, 2, TEMPER, true>
+                              : k_greedy_split<GREEDY_SPLIT_BLOCK, GREEDY_SPLIT_U, 2, TEMPER, false>)
+                 : (L.pen_any ? k_greedy_split<GREEDY_SPLIT_BLOCK, GREEDY_SPLIT_U, 1, TEMPER, true>
+                              : k_greedy_split<GREEDY_SPLIT_BLOCK, GREEDY_SPLIT_U, 1, TEMPER, false>);
     if (lds > 65536 && hipFuncSetAttribute((const void*)k,
                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)lds) != hipSuccess)
@@ -409,10 +430,14 @@ static int launch_argmax(const pz_launch& L, int n_rows, const int32_t* d_rows) 
   // static LDS: the block argmax scratch (2 words per wave)
   if (lds + kStatic > (size_t)L.max_lds) return -2;
   dim3 grid(n_rows), block(GREEDY_BLOCK);
-  auto k = vec ? (L.pen_any ? k_greedy<GREEDY_BLOCK, GREEDY_U, true, TEMPER, true>
-                            : k_greedy<GREEDY_BLOCK, GREEDY_U, true, TEMPER, false>)
-               : (L.pen_any ? k_greedy<GREEDY_BLOCK, GREEDY_U, false, TEMPER, true>
-                            : k_greedy<GREEDY_BLOCK, GREEDY_U, false, TEMPER, false>);
+  auto pick = [&](auto v) {
+    constexpr int VEC = decltype(v)::value;
+    return L.pen_any ? k_greedy<GREEDY_BLOCK, GREEDY_U, VEC, TEMPER, true>
+                     : k_greedy<GREEDY_BLOCK, GREEDY_U, VEC, TEMPER, false>;
+  };
+  auto k = vec == 2   ? pick(std::integral_constant<int, 2>())
+           : vec == 1 ? pick(std::integral_constant<int, 1>())
+                      : pick(std::integral_constant<int, 0>());
   if (lds > 65536 && hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)lds) != hipSuccess)
     return -1;

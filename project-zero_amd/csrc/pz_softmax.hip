@@ -215,7 +215,7 @@ __global__ __launch_bounds__(PZ_SP_BLOCK) void k_sm_walk(SmSplit A) {
 }
 
 // p = e * (1 / sum) for every score of the slice (NaN on degenerate rows).
-template <bool VI, bool VO>
+template <bool VI>
 __global__ __launch_bounds__(PZ_SP_BLOCK) PZ_SP_TWO_PER_CU void k_sm_write(SmSplit A) {
   __shared__ uint64_t etab[32];
   pz_etab_fill((pz_lds_u64*)etab);
@@ -249,13 +249,13 @@ __global__ __launch_bounds__(PZ_SP_BLOCK) PZ_SP_TWO_PER_CU void k_sm_write(SmSpl
 #pragma unroll
       for (int c = 0; c < 4; c++)
         v[c] = bad ? __builtin_nanf("") : pz_expf_tab(y[u][c] - rs.M, X.et) * rs.inv;
-      if (VO && i0 + 3 < len) {
-        pz_f4 q;
+      if (i0 + 3 < len) {
+        pz_f4u q;
         q.x = v[0];
         q.y = v[1];
         q.z = v[2];
         q.w = v[3];
-        *reinterpret_cast<pz_f4*>(o + i0) = q;
+        *reinterpret_cast<pz_f4u*>(o + i0) = q;
       } else {
 #pragma unroll
         for (int c = 0; c < 4; c++)
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(PZ_SP_BLOCK) PZ_SP_TWO_PER_CU void k_sm_write(SmSpl
   }
 }
 
-template <bool VI, bool VO>
+template <bool VI>
 int launch_split_t(pz_sampler* s, const SmSplit& A, int n_rows, size_t walk_lds) {
   auto kw = k_sm_walk<VI>;
   if (walk_lds > 65536 && hipFuncSetAttribute((const void*)kw,
@@ -276,7 +276,7 @@ int launch_split_t(pz_sampler* s, const SmSplit& A, int n_rows, size_t walk_lds)
   hipLaunchKernelGGL(k_sm_stat<VI>, grid, block, 0, s->stream, A);
   hipLaunchKernelGGL(k_sm_rec<VI>, grid, block, 0, s->stream, A);
   hipLaunchKernelGGL(kw, dim3(n_rows), block, walk_lds, s->stream, A);
-  hipLaunchKernelGGL((k_sm_write<VI, VO>), grid, block, 0, s->stream, A);
+  hipLaunchKernelGGL(k_sm_write<VI>, grid, block, 0, s->stream, A);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -316,11 +316,8 @@ int pz_launch_softmax_split(pz_sampler* s, const PzSplitWs& ws, const float* d_i
   A.nc = nc;
   const size_t walk_lds = pz_sp_walk_lds(pl.nseg, nc);
   const bool vi = (ld_in % 4 == 0) && (((uintptr_t)d_in & 15) == 0);
-  const bool vo = (ld_out % 4 == 0) && (((uintptr_t)d_out & 15) == 0);
-  if (vi) return vo ? launch_split_t<true, true>(s, A, n_rows, walk_lds)
-                    : launch_split_t<true, false>(s, A, n_rows, walk_lds);
-  return vo ? launch_split_t<false, true>(s, A, n_rows, walk_lds)
-            : launch_split_t<false, false>(s, A, n_rows, walk_lds);
+  return vi ? launch_split_t<true>(s, A, n_rows, walk_lds)
+            : launch_split_t<false>(s, A, n_rows, walk_lds);
 }
 
 int pz_launch_softmax_rows(pz_sampler* s, const float* d_in, long ld_in, float* d_out,

@@ -705,7 +705,7 @@ __global__ __launch_bounds__(BLOCK) void k_topk_split(
   const int hi = lo + PZ_TILE < V ? lo + PZ_TILE : V;
   const int e0 = lo + 4 * tid;
   float a[4];
-  const int n = pz_load4<VEC, false>(x, hi, e0, a);
+  const int n = pz_load4_once<VEC>(x, hi, e0, a);
   const uint64_t tab = tid < 32 ? pz_exp2_tab[tid] : 0ull;
   // the uniform: from the launch's arguments for the first rows of a small
   // batch (no memory read on the merge's path), else from u
