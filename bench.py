@@ -589,7 +589,7 @@ def run_attention(args, torch, cpu):
         e = {"ctx": ctx, "kernel_us": kern * 1e3, "achieved_gbs": gbs, "frac": gbs / HBM_PEAK_GBS,
              "distinct_blocks": nrot,
              "kernel": ("k_attn_wave" if ctx <= 1024 else "k_attn_row" if ctx <= 8192 else
-                        "k_attn_stat + k_attn_rec + k_attn_walk + k_attn_write (row split)")}
+                        "k_sm_stat + k_sm_rec + k_sm_walk + k_sm_write (row split)")}
         if cpu.enabled:
             s.sync()
             got = t_o[:heads].cpu().numpy()
