@@ -37,6 +37,7 @@
 #include "pz_exact.h"
 #include "pz_launch.h"
 #include "pz_rowpass.h"
+#include "pz_sampler_impl.h"
 #include "pz_split.h"
 
 namespace {
@@ -136,6 +137,8 @@ struct CatArgs {
   int32_t* ids_out;
   float* p_out;
   PzSplitWs ws;
+  uint64_t* state;  // RNG states to draw from into u_out (or null: u is there already)
+  float* u_out;
   int nseg, spw, S, nc;
   int est_abs;  // seg_s holds the front pass's absolute estimates
 };
@@ -151,6 +154,17 @@ __device__ __forceinline__ PzRow<VEC> cat_row(const CatArgs& A, int row, char* l
   const int32_t* hrow = A.hist ? A.hist + (long)row * A.H : nullptr;
   pz_penalty_build_range<PZ_SP_BLOCK>(R.P, lds, A.V, lo, hi, A.hcap, hrow, A.H, prm);
   return R;
+}
+
+// A decode step's draw of the row (generate.c:159: every categorical row
+// draws once), by the first launch's first slice, for k_cat_draw: a launch of
+// its own took 2-4 us before the others.
+__device__ __forceinline__ void cat_step_draw(const CatArgs& A, int row) {
+  if (A.state && blockIdx.x == 0 && threadIdx.x == 0) {
+    uint64_t s = A.state[row];
+    A.u_out[row] = pz_rng_float(s);
+    A.state[row] = s;
+  }
 }
 
 // softmax.c:4-23 gives NaN everywhere when any y is NaN or the maximum is not
@@ -172,6 +186,7 @@ __global__ __launch_bounds__(PZ_SP_BLOCK) PZ_SP_TWO_PER_CU void k_cat_front(CatA
   pz_etab_fill((pz_lds_u64*)etab);
   const int row = pz_row_of(A.rows, blockIdx.y);
   const PzSlice sl = pz_sp_slice(A.nseg, A.spw);
+  cat_step_draw(A, row);
   if (threadIdx.x == 0) {
     SS.any = 0u;
     F.fail = 0;
@@ -188,6 +203,7 @@ __global__ __launch_bounds__(PZ_SP_BLOCK) PZ_SP_TWO_PER_CU void k_cat_stat(CatAr
   __shared__ PzSpShared SS;
   const int row = pz_row_of(A.rows, blockIdx.y);
   const PzSlice sl = pz_sp_slice(A.nseg, A.spw);
+  cat_step_draw(A, row);
   if (threadIdx.x == 0) SS.any = 0u;
   const PzRow<VEC> R = cat_row<VEC>(A, row, lds, pz_sp_lo(sl), pz_sp_hi(sl, A.V));
   __syncthreads();
@@ -410,6 +426,8 @@ int launch_cat_split(const pz_launch& L, int n_rows, const int32_t* d_rows) {
   A.H = L.H;
   A.hcap = L.hcap;
   A.u = L.u;
+  A.state = L.step_state;
+  A.u_out = L.step_u;
   A.ids_out = L.ids;
   A.p_out = L.p_out;
   A.ws = ws;
@@ -452,5 +470,6 @@ int pz_launch_categorical(const pz_launch& L, int n_rows, const int32_t* d_rows)
   const int rc = vec ? launch_cat_split<true>(L, n_rows, d_rows)
                      : launch_cat_split<false>(L, n_rows, d_rows);
   if (rc != -2) return rc;
+  if (L.step_state && pz_launch_step_draw(L, L.B, L.step_state, L.step_u) != 0) return -1;
   return vec ? launch_cat_t<true>(L, n_rows, d_rows) : launch_cat_t<false>(L, n_rows, d_rows);
 }

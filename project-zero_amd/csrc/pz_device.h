@@ -130,6 +130,18 @@ __device__ __forceinline__ void pz_lds_barrier() {
 // kernels' code size beyond the instruction cache.
 __device__ __noinline__ float pz_expf(float x) { return pz_expf_inline(x); }
 
+// rng.c:8-17: xorshift64*; the product's upper 31 bits over 2^31.  The
+// value is below 2^31, so converting it through uint32 (v_cvt_f32_u32,
+// round to nearest even) equals the reference's 64-bit int -> float
+// conversion; the division by 2^31 is exact.
+__device__ __forceinline__ float pz_rng_float(uint64_t& s) {
+  s ^= s >> 12;
+  s ^= s << 25;
+  s ^= s >> 27;
+  const uint32_t hi = (uint32_t)((s * 0x2545F4914F6CDD1DULL) >> 33);
+  return (float)hi / 2147483648.0f;
+}
+
 // ---------------------------------------------------------------------------
 // Order key: monotone uint32 image of an fp32 value (larger value -> larger
 // key), with -0.0 folded onto +0.0 so the two compare equal exactly as the

@@ -49,6 +49,8 @@ struct pz_launch {
   bool temp_div;        // temperature as x / T (scalar build) rather than x * (1/T)
   const float* u;       // device [B] uniforms
   const float* h_u = nullptr;  // host copy of the same uniforms, when the caller has one
+  uint64_t* step_state = nullptr;  // a decode step of categorical rows only: the RNG states
+  float* step_u = nullptr;         // that the sampling launch draws from, into step_u (== u)
   int B = 0;            // rows of the call
   int32_t* ids;         // device [B] sampled ids
   float* p_out;         // device [B] p(chosen) or nullptr

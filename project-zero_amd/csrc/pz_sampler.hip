@@ -371,7 +371,13 @@ int pz_dispatch_resolved(pz_sampler* s, const float* d_logits, int B, int V, lon
   L.n_cu = s->n_cu;
   L.stream = s->stream;
 
-  if (hooks && pz_launch_step_draw(L, B, hooks->state, s->d_u_step) != 0)
+  // the step's draws: none for greedy rows, by the sampling launch itself when
+  // every row is categorical, else a launch of their own
+  if (hooks && count[PZ_MODE_CATEGORICAL] == B) {
+    L.step_state = hooks->state;
+    L.step_u = s->d_u_step;
+  } else if (hooks && count[PZ_MODE_GREEDY] != B &&
+             pz_launch_step_draw(L, B, hooks->state, s->d_u_step) != 0)
     return fail(s, PZ_EDEVICE, "launch of the step draw failed");
   int m = -1;
   const int rc = pz_launch_modes(L, count, offset, modes_present, s->d_rows, &m);

@@ -20,18 +20,6 @@
 
 namespace {
 
-// rng.c:8-17: xorshift64*; the product's upper 31 bits over 2^31.  The
-// value is below 2^31, so converting it through uint32 (v_cvt_f32_u32,
-// round to nearest even) equals the reference's 64-bit int -> float
-// conversion; the division by 2^31 is exact.
-__device__ __forceinline__ float step_rng_float(uint64_t& s) {
-  s ^= s >> 12;
-  s ^= s << 25;
-  s ^= s >> 27;
-  const uint32_t hi = (uint32_t)((s * 0x2545F4914F6CDD1DULL) >> 33);
-  return (float)hi / 2147483648.0f;
-}
-
 // The value the chain sees for id 0 of row b (penalties as the kernels
 // apply them, then temperature): top_p.c starts its maximum at the row's
 // first element, so a NaN there leaves no candidate and the row returns
@@ -81,7 +69,7 @@ __global__ void k_step_draw(const float* logits, long ld, int V, int B,
   float r = 0.0f;
   if (draws) {
     uint64_t s = state[b];
-    r = step_rng_float(s);
+    r = pz_rng_float(s);
     state[b] = s;
   }
   u[b] = r;

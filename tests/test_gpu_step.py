@@ -148,3 +148,35 @@ def test_top_p_above_vocabulary_guard_does_not_draw(torch_cuda):
         draws, _ = run_steps(torch_cuda, s, batches, [pz.row_params(temperature=0.7, top_p=0.9)],
                              seeds, [], n_steps=4, label="guard")
     assert draws == 0
+
+
+# one slice, several slices in the front launch, more rows than its one round
+# holds (the separate statistics launch), a vocabulary past the split's LDS
+# (one workgroup per row, the draws in a launch of their own)
+@pytest.mark.parametrize("B,V,H", [(1, 300, 0), (5, 20001, 0), (48, 50257, 0), (600, 9000, 0),
+                                   (700, 1000, 16), (2, 700000, 0)])
+def test_categorical_steps_draw_in_the_sampling_launch(torch_cuda, B, V, H):
+    print(f"case step categorical B={B} V={V} H={H}", flush=True)
+    rng = np.random.default_rng(B + V)
+    n = 2 if V < 100000 else 1
+    batches = [(rng.standard_normal((B, V), dtype=np.float32) * 2.0) for _ in range(n)]
+    if B > 4:
+        batches[0][3, 7] = np.nan  # the draw falls back to V - 1, after drawing
+    hist = rng.integers(0, V, (B, H)).astype(np.int32) if H else None
+    seeds = np.arange(1, B + 1, dtype=np.uint64) * np.uint64(7368787)
+    params = [pz.row_params(temperature=0.9, rep_penalty=1.2 if H else 1.0)]
+    with pz.Sampler(B, V, max_hist=max(H, 1)) as s:
+        draws, _ = run_steps(torch_cuda, s, batches, params, seeds, [3, V - 1], hist=hist,
+                             n_steps=3 if n > 1 else 2, label="categorical")
+    assert draws == B * (3 if n > 1 else 2)
+
+
+def test_greedy_steps_do_not_draw(torch_cuda):
+    B, V = 9, 4097
+    print(f"case step greedy B={B} V={V}", flush=True)
+    x = pz.synth_normal(B, V, 3.0, 0xE77)
+    seeds = np.arange(1, B + 1, dtype=np.uint64)
+    with pz.Sampler(B, V) as s:
+        draws, _ = run_steps(torch_cuda, s, [x], [pz.row_params(temperature=0.0)], seeds, [3],
+                             n_steps=2, label="greedy")
+    assert draws == 0
