@@ -139,6 +139,7 @@ struct CatArgs {
   PzSplitWs ws;
   uint64_t* state;  // RNG states to draw from into u_out (or null: u is there already)
   float* u_out;
+  PzEosCheck eos;
   int nseg, spw, S, nc;
   int est_abs;  // seg_s holds the front pass's absolute estimates
 };
@@ -342,7 +343,9 @@ __global__ __launch_bounds__(CAT_WALK_BLOCK) void k_cat_draw(CatArgs A, int pen_
   const PzRowState rs = A.ws.rs[row];
   if (cat_bad(rs.flags)) {
     if (threadIdx.x == 0) {
-      A.ids_out[row] = (rs.flags & PZ_RS_FAILED) ? PZ_ID_FAILED : A.V - 1;
+      const int id = (rs.flags & PZ_RS_FAILED) ? PZ_ID_FAILED : A.V - 1;
+      A.ids_out[row] = id;
+      pz_eos_mark(A.eos, row, id);
       if (A.p_out) A.p_out[row] = __builtin_nanf("");
     }
     return;
@@ -373,6 +376,7 @@ __global__ __launch_bounds__(CAT_WALK_BLOCK) void k_cat_draw(CatArgs A, int pen_
   if (threadIdx.x == 0) {
     const int id = hit_sh >= 0 ? hit_sh : A.V - 1;
     A.ids_out[row] = id;
+    pz_eos_mark(A.eos, row, id);
     if (A.p_out) {
       float yy[4];
       const int e0 = id & ~3;
@@ -428,6 +432,7 @@ int launch_cat_split(const pz_launch& L, int n_rows, const int32_t* d_rows) {
   A.u = L.u;
   A.state = L.step_state;
   A.u_out = L.step_u;
+  A.eos = L.eos;
   A.ids_out = L.ids;
   A.p_out = L.p_out;
   A.ws = ws;
@@ -471,5 +476,8 @@ int pz_launch_categorical(const pz_launch& L, int n_rows, const int32_t* d_rows)
                      : launch_cat_split<false>(L, n_rows, d_rows);
   if (rc != -2) return rc;
   if (L.step_state && pz_launch_step_draw(L, L.B, L.step_state, L.step_u) != 0) return -1;
-  return vec ? launch_cat_t<true>(L, n_rows, d_rows) : launch_cat_t<false>(L, n_rows, d_rows);
+  const int r = vec ? launch_cat_t<true>(L, n_rows, d_rows) : launch_cat_t<false>(L, n_rows, d_rows);
+  if (r == 0 && L.eos.out)
+    return pz_launch_step_eos(L.stream, L.ids, L.B, L.eos.ids, L.eos.n, L.eos.out);
+  return r;
 }

@@ -142,6 +142,20 @@ __device__ __forceinline__ float pz_rng_float(uint64_t& s) {
   return (float)hi / 2147483648.0f;
 }
 
+// generate.c:198-211: a decode step's EOS flag of a row, written with its id
+// (out null: no flags asked for, or a launch of their own writes them).
+struct PzEosCheck {
+  const int32_t* ids = nullptr;
+  int n = 0;
+  uint8_t* out = nullptr;
+};
+__device__ __forceinline__ void pz_eos_mark(const PzEosCheck& E, int row, int32_t id) {
+  if (!E.out) return;
+  uint8_t f = 0;
+  for (int e = 0; e < E.n; e++) f |= (uint8_t)(E.ids[e] == id);
+  E.out[row] = f;
+}
+
 // ---------------------------------------------------------------------------
 // Order key: monotone uint32 image of an fp32 value (larger value -> larger
 // key), with -0.0 folded onto +0.0 so the two compare equal exactly as the

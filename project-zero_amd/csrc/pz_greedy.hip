@@ -134,7 +134,7 @@ __global__ __launch_bounds__(BLOCK) void k_greedy(
     const float* __restrict__ logits, long ld, int V,
     const int32_t* __restrict__ rows, const pz_row_params_dev* __restrict__ params,
     int n_params, const int32_t* __restrict__ hist, int H, int hcap,
-    int32_t* __restrict__ ids_out, float* __restrict__ p_out) {
+    int32_t* __restrict__ ids_out, float* __restrict__ p_out, PzEosCheck eos) {
   extern __shared__ __align__(16) char lds[];
   __shared__ float red_v[BLOCK / PZ_WAVE];
   __shared__ int red_i[BLOCK / PZ_WAVE];
@@ -225,6 +225,7 @@ __global__ __launch_bounds__(BLOCK) void k_greedy(
     if (y0 != y0 || bi == 0x7fffffff) bi = 0;
     ids_out[row] = bi;
     if (p_out) p_out[row] = 1.0f;
+    pz_eos_mark(eos, row, bi);
   }
 }
 
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(BLOCK) void k_greedy_split(
     const int32_t* __restrict__ rows, const pz_row_params_dev* __restrict__ params,
     int n_params, const int32_t* __restrict__ hist, int H, int hcap,
     int32_t* __restrict__ ids_out, float* __restrict__ p_out, uint64_t* __restrict__ words,
-    int wstride, uint32_t* __restrict__ arrive, uint32_t cap) {
+    int wstride, uint32_t* __restrict__ arrive, uint32_t cap, PzEosCheck eos) {
   extern __shared__ __align__(16) char lds[];
   __shared__ float red_v[BLOCK / PZ_WAVE];
   __shared__ int red_i[BLOCK / PZ_WAVE];
@@ -355,9 +356,12 @@ __global__ __launch_bounds__(BLOCK) void k_greedy_split(
   const bool all_seen = __builtin_amdgcn_ballot_w64(!seen) == 0ull;
   if (tid == 0) {
     // no candidate (every value NaN or -inf): the scan ends on index 0
-    ids_out[row] = !all_seen ? PZ_ID_FAILED : (k == 1ull || k == ~0ull) ? 0
-                                                                      : (int32_t)~(uint32_t)k;
+    const int32_t id = !all_seen                     ? PZ_ID_FAILED
+                       : (k == 1ull || k == ~0ull) ? 0
+                                                   : (int32_t)~(uint32_t)k;
+    ids_out[row] = id;
     if (p_out) p_out[row] = 1.0f;
+    pz_eos_mark(eos, row, id);
     __hip_atomic_store(&arrive[row], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
@@ -423,7 +427,7 @@ static int launch_argmax(const pz_launch& L, int n_rows, const int32_t* d_rows) 
     hipLaunchKernelGGL(k, dim3(S, n_rows), dim3(GREEDY_SPLIT_BLOCK), lds, L.stream, L.logits,
                        L.ld,
                        L.V, chunk, d_rows, L.params, L.n_params, L.hist, L.H, L.hcap, L.ids,
-                       L.p_out, L.ws.meet, 2 * L.ws.smax, L.ws.arrive, L.wait_polls);
+                       L.p_out, L.ws.meet, 2 * L.ws.smax, L.ws.arrive, L.wait_polls, L.eos);
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
   const size_t lds = L.pen_any ? pz_penalty_lds_bytes(L.V, L.hcap) : 0;
@@ -442,7 +446,7 @@ static int launch_argmax(const pz_launch& L, int n_rows, const int32_t* d_rows) 
                                          (int)lds) != hipSuccess)
     return -1;
   hipLaunchKernelGGL(k, grid, block, lds, L.stream, L.logits, L.ld, L.V, d_rows, L.params,
-                     L.n_params, L.hist, L.H, L.hcap, L.ids, L.p_out);
+                     L.n_params, L.hist, L.H, L.hcap, L.ids, L.p_out, L.eos);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -4,6 +4,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "pz_device.h"
 #include "pz_params.h"
 #include "pz_sampler.h"
 #include "pz_split.h"
@@ -51,6 +52,8 @@ struct pz_launch {
   const float* h_u = nullptr;  // host copy of the same uniforms, when the caller has one
   uint64_t* step_state = nullptr;  // a decode step of categorical rows only: the RNG states
   float* step_u = nullptr;         // that the sampling launch draws from, into step_u (== u)
+  PzEosCheck eos;       // a decode step of rows of one mode, greedy or categorical: its EOS
+                        // flags, written by the launch that writes the ids
   int B = 0;            // rows of the call
   int32_t* ids;         // device [B] sampled ids
   float* p_out;         // device [B] p(chosen) or nullptr

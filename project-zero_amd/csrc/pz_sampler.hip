@@ -379,12 +379,20 @@ int pz_dispatch_resolved(pz_sampler* s, const float* d_logits, int B, int V, lon
   } else if (hooks && count[PZ_MODE_GREEDY] != B &&
              pz_launch_step_draw(L, B, hooks->state, s->d_u_step) != 0)
     return fail(s, PZ_EDEVICE, "launch of the step draw failed");
+  // the EOS flags with the ids where one kind of launch writes them all
+  const bool eos_here =
+      hooks && (count[PZ_MODE_CATEGORICAL] == B || count[PZ_MODE_GREEDY] == B);
+  if (eos_here && hooks->eos_out) {
+    L.eos.ids = s->d_eos;
+    L.eos.n = s->n_eos;
+    L.eos.out = hooks->eos_out;
+  }
   int m = -1;
   const int rc = pz_launch_modes(L, count, offset, modes_present, s->d_rows, &m);
   if (rc == -2) return fail(s, PZ_ENOTSUP, "sampling mode %d not supported for V=%d", m, V);
   if (rc != 0) return fail(s, PZ_EDEVICE, "launch of mode %d failed: %s", m,
                            hipGetErrorString(hipGetLastError()));
-  if (hooks && hooks->eos_out &&
+  if (hooks && hooks->eos_out && !eos_here &&
       pz_launch_step_eos(s->stream, d_ids, B, s->d_eos, s->n_eos, hooks->eos_out) != 0)
     return fail(s, PZ_EDEVICE, "launch of the EOS check failed");
   return PZ_OK;
