@@ -7,7 +7,9 @@
 // with the model's EOS ids (generate.c:198-211).  Here the states are a
 // device array, one per row, and a step is three launches on the sampler's
 // stream: the draw (k_step_draw, one thread per row), the batched sampler
-// reading the uniforms it wrote, and the EOS flags (k_step_eos).
+// reading the uniforms it wrote, and the EOS flags (k_step_eos).  Batches of
+// one kind need fewer: greedy rows draw nothing, categorical rows draw in
+// their first launch, and both write the flags with the ids.
 #include <hip/hip_runtime.h>
 
 #include <string.h>
