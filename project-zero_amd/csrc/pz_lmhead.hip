@@ -214,6 +214,13 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
 //   * Bounds: above about 64 batch rows the three parts' 6 V n B operations
 //     (1.3 PFLOP/s at 256 rows, against 1.65 for a large library bf16 product
 //     on the same card), below that one read of W.
+//   * Every tile adds up k in the same order (32 k at a time from 0, the
+//     smallest part first), so a logit depends on its row of W and its
+//     activations alone: equal rows of W tie wherever they lie, and a batch
+//     row's logits are the same in any batch.  (Row tiles that each start k
+//     at another stage spread rows a multiple of 4 KiB apart over the memory
+//     channels, 16 batch rows at 160000 x 2048 in 126 us instead of 166, but
+//     give equal rows different sums.)
 // Workgroups of one row tile (its batch blocks) are consecutive on one XCD,
 // so its L2 serves W to all but the first.
 // MODE 1 (argmax keys) as in k_lmhead.
@@ -324,14 +331,7 @@ k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __re
   const int klast = (nst - 1) * 32 * KS + 8 * piece;
   const uint32_t wadj = klast < n ? 0u : (uint32_t)(klast - (n - 8)) * 2u;
   const uint32_t xoff = (uint32_t)lane * 16u;
-  // where this workgroup starts in k (it wraps): rows a multiple of 4 KiB
-  // apart put the same k of every row on the same few memory channels, so
-  // the row tiles each start one stage further on (16 batch rows at 160000 x
-  // 2048: 166 -> 126 us, at 80000 x 4096: 182 -> 142 us; other row lengths,
-  // and the tiles the matrix cores bound, gain nothing and start at 0)
-  const int rot = CF <= 4 && n % 2048 == 0 ? (row0 >> 8) % nst : 0;
-  auto issue = [&](int cc, int buf, int i) {  // load i of the cc-th stage into ring slot buf
-    const int c = cc + rot < nst ? cc + rot : cc + rot - nst;
+  auto issue = [&](int c, int buf, int i) {  // load i of stage c into ring slot buf
     const uint32_t l0 = lds0 + (uint32_t)buf * STG * 2;
     if (i < WPW) {
       const uint32_t off = woff[i] - (c == nst - 1 ? wadj : 0u), to = l0 + (w * WPW + i) * 1024;

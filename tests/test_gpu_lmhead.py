@@ -199,3 +199,30 @@ def test_lm_head_matrix_core_tiles(torch_cuda, B, V, n):
     tol = n * 2.0 ** -24 * bound + 1e-30
     print(f"B{B} V{V} n{n}: max |err| / bound = {float((err / tol).max()):.4f}", flush=True)
     assert (err <= tol).all()
+
+
+# row lengths around the multiples of 2048 (rows of W a multiple of 4 KiB
+# apart), batches in every tile of the GEMM and in more than one chunk
+@pytest.mark.parametrize("n", [2048, 2056, 2560, 4096, 6144])
+def test_equal_rows_give_equal_logits(torch_cuda, n):
+    """From four batch rows on, a logit depends on its row of W and its
+    activations alone: not on where the row lies in the vocabulary, on the
+    batch row or on the batch.  Equal rows of W in different row tiles tie, so
+    the fused argmax returns the lowest of their ids."""
+    torch = torch_cuda
+    rng = np.random.default_rng(n)
+    period, V = 200, 1100
+    base = bf16_bits(rng.standard_normal((period, n), dtype=np.float32) * 0.02)
+    wb = np.ascontiguousarray(np.tile(base, (V // period + 1, 1))[:V])
+    x7 = rng.standard_normal((7, n), dtype=np.float32)
+    first = None
+    with pz.Sampler(300, V) as s:
+        for B in (4, 16, 40, 64, 100, 130, 256, 300):
+            print(f"case lmhead equal rows n={n} B={B}", flush=True)
+            logits, ids, gids = run(torch, wb, np.ascontiguousarray(x7[np.arange(B) % 7]), s)
+            bits = logits.view(np.int32)
+            if first is None:
+                first = run(torch, base, x7, s)[0].view(np.int32)
+            want = first[np.arange(B) % 7][:, np.arange(V) % period]
+            assert (bits == want).all(), (B, np.argwhere(bits != want)[:3])
+            assert (ids < period).all() and (gids == ids).all()
