@@ -208,6 +208,10 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
 //     XOR with the row in the source address so that the fragment reads do
 //     not meet in the banks.  The 256 x 256 tile's stage only fits with
 //     KS = 1; it is bound by the matrix cores, not by that.
+//   * NS = 0: no workspace, ring or stages -- a wave reads its tiles of W and
+//     splits its batch rows' activations in registers, KS k-steps ahead -- for
+//     rows longer than the workspace serves (16 batch rows at 4000 x 131080:
+//     3.2 ms, 3.7 where every workgroup staged the parts in LDS).
 //   * 128256 x 2560: 16 batch rows 112 us, 32 124, 64 167, 128 237, 256 405
 //     (one launch per 32 rows that split the activations in every workgroup
 //     took 143, 152, 301, 601 and 1203).
@@ -235,22 +239,15 @@ __device__ __forceinline__ float lm_bf16_f(uint16_t h) { return __uint_as_float(
 // workgroups' atomics do not all meet on the batch's few words.
 constexpr int LMM_SLOTS = 16;
 
-// The activations' three bf16 parts as fragments: part p of batch rows 16 ct
-// .. +15 and k 32 ks .. +31 at xp[((ks * ctt + ct) * 3 + p) * LMX_FRAG]
-// (zeros past nb and past n).  One wave per (ks, ct).
-__global__ __launch_bounds__(64) void k_lmx_split(const float* __restrict__ X, long ldx, int nb,
-                                                  int n, int ctt, uint16_t* __restrict__ xp) {
-  const int ks = blockIdx.x, ct = blockIdx.y, lane = threadIdx.x;
-  const int b = ct * 16 + (lane & 15), k0 = ks * 32 + 8 * (lane >> 4);
-  uint32_t h[3][4];
+// The three bf16 parts of 8 activations, two to a word.
+__device__ __forceinline__ void lm_split8(const float (&x)[8], lm_u32x4 (&h)[3]) {
 #pragma unroll
   for (int e = 0; e < 8; e++) {
-    const float x = b < nb && k0 + e < n ? X[(size_t)b * ldx + k0 + e] : 0.0f;
-    const uint32_t ux = __float_as_uint(x);
+    const uint32_t ux = __float_as_uint(x[e]);
     const bool fin = (ux & 0x7f800000u) != 0x7f800000u;
     // (a NaN whose payload sits in the low bits stays a NaN)
     const uint32_t h0 = fin || !(ux & 0x7fffffu) ? ux >> 16 : 0x7fc0u;
-    const float r0 = fin ? x - __uint_as_float(h0 << 16) : 0.0f;  // exact: the low 16 bits
+    const float r0 = fin ? x[e] - __uint_as_float(h0 << 16) : 0.0f;  // exact: the low 16 bits
     const uint32_t h1 = __float_as_uint(r0) >> 16;
     const float r1 = r0 - __uint_as_float(h1 << 16);  // exact: at most 8 significant bits left
     const uint32_t h2 = __float_as_uint(r1) >> 16;
@@ -258,10 +255,24 @@ __global__ __launch_bounds__(64) void k_lmx_split(const float* __restrict__ X, l
 #pragma unroll
     for (int p = 0; p < 3; p++) h[p][e >> 1] = e & 1 ? h[p][e >> 1] | hs[p] << 16 : hs[p];
   }
+}
+
+// The activations' three bf16 parts as fragments: part p of batch rows 16 ct
+// .. +15 and k 32 ks .. +31 at xp[((ks * ctt + ct) * 3 + p) * LMX_FRAG]
+// (zeros past nb and past n).  One wave per (ks, ct).
+__global__ __launch_bounds__(64) void k_lmx_split(const float* __restrict__ X, long ldx, int nb,
+                                                  int n, int ctt, uint16_t* __restrict__ xp) {
+  const int ks = blockIdx.x, ct = blockIdx.y, lane = threadIdx.x;
+  const int b = ct * 16 + (lane & 15), k0 = ks * 32 + 8 * (lane >> 4);
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) x[e] = b < nb && k0 + e < n ? X[(size_t)b * ldx + k0 + e] : 0.0f;
+  lm_u32x4 h[3];
+  lm_split8(x, h);
   uint16_t* o = xp + ((size_t)ks * ctt + ct) * 3 * LMX_FRAG + lane * 8;
 #pragma unroll
   for (int p = 0; p < 3; p++)
-    *reinterpret_cast<lm_u32x4*>(o + p * LMX_FRAG) = lm_u32x4{h[p][0], h[p][1], h[p][2], h[p][3]};
+    *reinterpret_cast<lm_u32x4*>(o + p * LMX_FRAG) = h[p];
 }
 
 // 16 bytes per lane from base + off to LDS at byte address lds + 16 lane.
@@ -300,10 +311,11 @@ k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __re
   constexpr int WI = RF * KS, XF = CF * 3 * KS;  // 1 KiB loads of a stage: weights, parts
   constexpr int WPW = WI / NW, XPW = (XF + NW - 1) / NW, PER = WPW + XPW;  // of a wave
   constexpr int STG = (WI + XF) * LMX_FRAG;
-  static_assert(WI % NW == 0 && (KS == 1 || KS == 2) && (NS & 1) + NS > 1, "");
+  static_assert(WI % NW == 0 && (KS == 1 || KS == 2) && (NS == 0 || NS >= 2), "");
   static_assert(TR % WC == 0 || WC % TR == 0, "");
-  static_assert((size_t)NS * STG * 2 >= NW * CF * 16 * 8, "the epilogue's keys reuse the ring");
-  __shared__ __align__(16) uint16_t sh[NS * STG];
+  constexpr int SH = NS ? NS * STG : NW * CF * 64;
+  static_assert((size_t)SH * 2 >= NW * CF * 16 * 8, "the epilogue's keys reuse the ring");
+  __shared__ __align__(16) uint16_t sh[SH];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, g = lane >> 4;
   const int wr = w % WR, wc = w / WR;
@@ -313,37 +325,6 @@ k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __re
   const int rt = (slot / ncb) * 8 + (blockIdx.x & 7), cb = slot % ncb;
   if (rt >= nrt) return;
   const int row0 = rt * RF * 16;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)sh;
-  const uint16_t* wbase = W + (size_t)row0 * n;
-  const int nst = (n + 32 * KS - 1) / (32 * KS);
-  // this wave's loads of W: row and 16-byte piece per lane.  Rows past V read
-  // row V - 1 (values unused); pieces past n read the row's last piece, which
-  // meets zero parts (and is non-finite only in a row flagged anyway).
-  uint32_t woff[WPW];
-  const int piece = KS == 1 ? g : (lane & 7) ^ (lane >> 3);
-#pragma unroll
-  for (int i = 0; i < WPW; i++) {
-    const int q = w * WPW + i;
-    const int r = KS == 1 ? q * 16 + m : q * 8 + (lane >> 3);
-    const int last = V - 1 - row0;
-    woff[i] = ((uint32_t)(r < last ? r : last) * (uint32_t)n + 8u * piece) * 2u;
-  }
-  const int klast = (nst - 1) * 32 * KS + 8 * piece;
-  const uint32_t wadj = klast < n ? 0u : (uint32_t)(klast - (n - 8)) * 2u;
-  const uint32_t xoff = (uint32_t)lane * 16u;
-  auto issue = [&](int c, int buf, int i) {  // load i of stage c into ring slot buf
-    const uint32_t l0 = lds0 + (uint32_t)buf * STG * 2;
-    if (i < WPW) {
-      const uint32_t off = woff[i] - (c == nst - 1 ? wadj : 0u), to = l0 + (w * WPW + i) * 1024;
-      lm_lds_load16<NT>(wbase + c * 32 * KS, off, to);
-    } else {
-      int q = w * XPW + i - WPW;
-      if (XF % NW) q = q < XF ? q : XF - 1;  // (the same bytes to the same place again)
-      const int s = q / (CF * 3), e = q - s * CF * 3;
-      lm_lds_load16<false>(xp + (((size_t)(c * KS + s) * ctt + cb * CF) * 3 + e) * LMX_FRAG, xoff,
-                    l0 + (WI + q) * 1024);
-    }
-  };
   lm_f32x4 acc[TR][TC];
 #pragma unroll
   for (int t = 0; t < TR; t++)
@@ -352,71 +333,172 @@ k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __re
   // largest |weight| bits seen, two halves; the waves that share rows take
   // their tiles in turn
   lm_u16x2 wmax = {0, 0};
+  if constexpr (NS == 0) {
+    // no ring: a wave's own loads, KS k-steps ahead, its batch rows' parts
+    // made in registers
+    static_assert(NS > 0 || WC == 1, "");
+    const uint16_t* wp[TR];
 #pragma unroll
-  for (int i = 0; i < NS - 1; i++)
-#pragma unroll
-    for (int q = 0; q < PER; q++) issue(i < nst ? i : nst - 1, i, q);
-  int buf = 0, nbuf = NS - 1;
-#pragma clang loop unroll(disable)
-  for (int c = 0; c < nst; c++) {
-    // stage c has arrived (the NS - 2 after it may be on their way), in every
-    // wave; and every wave is done reading the slot that is filled next
-    lm_wait<(NS - 2) * PER>();
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    const uint16_t* sw = sh + buf * STG;
-    const uint16_t* sx = sw + WI * LMX_FRAG;
-    const int cn = c + NS - 1 < nst ? c + NS - 1 : nst - 1;  // (past the end: reloaded, unused)
-#pragma unroll
-    for (int s = 0; s < KS; s++) {
-      lm_bf16x8 a[TR], b[3][TC];
-      const uint16_t* sxs = sx + (s * CF + wc * TC) * 3 * LMX_FRAG + lane * 8;
-#pragma unroll
-      for (int j = 0; j < TC; j++)
-        b[2][j] = *reinterpret_cast<const lm_bf16x8*>(sxs + (j * 3 + 2) * LMX_FRAG);
-#pragma unroll
-      for (int t = 0; t < TR; t++)
-        a[t] = *reinterpret_cast<const lm_bf16x8*>(
-            KS == 1 ? sw + (wr * TR + t) * LMX_FRAG + lane * 8
-                    : sw + (wr * TR + t) * 2 * LMX_FRAG + m * 64 + ((s * 4 + g) ^ (m & 7)) * 8);
-#pragma unroll
-      for (int p = 1; p >= 0; p--)
-#pragma unroll
-        for (int j = 0; j < TC; j++)
-          b[p][j] = *reinterpret_cast<const lm_bf16x8*>(sxs + (j * 3 + p) * LMX_FRAG);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int p = 2; p >= 0; p--)
-#pragma unroll
-        for (int j = 0; j < TC; j++)
-#pragma unroll
-          for (int t = 0; t < TR; t++) {
-            acc[t][j] =
-                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[p][j], acc[t][j], 0, 0, 0);
-            // the next stage's loads, one every few MFMAs of the first k-step
-            constexpr int SP = 3 * TR * TC / PER >= 4 ? 4 : 3 * TR * TC / PER;
-            static_assert(SP >= 1, "");
-            const int q = ((2 - p) * TC + j) * TR + t;
-            if (s == 0 && q % SP == SP - 1 && q / SP < PER) {
-              issue(cn, nbuf, q / SP);
-              __builtin_amdgcn_sched_barrier(0);
-            }
-          }
-#pragma unroll
-      for (int t = 0; t < TR; t++)
-        if (WC == 1 || t % WC == wc % TR) {
-          const lm_u32x4 q = __builtin_bit_cast(lm_u32x4, a[t]);
-#pragma unroll
-          for (int e = 0; e < 4; e++)
-            wmax = __builtin_elementwise_max(wmax,
-                                             __builtin_bit_cast(lm_u16x2, q[e] & 0x7fff7fffu));
-        }
+    for (int t = 0; t < TR; t++) {
+      const int r = row0 + (wr * TR + t) * 16 + m;
+      wp[t] = W + (size_t)(r < V ? r : V - 1) * n;  // rows past V: a valid row, result unused
     }
-    asm volatile("" ::: "memory");
-    buf = buf + 1 == NS ? 0 : buf + 1;
-    nbuf = nbuf + 1 == NS ? 0 : nbuf + 1;
+    lm_u32x4 aw[KS][TR];
+    pz_f4u xa[KS][TC][2];
+    auto fetch = [&](int k0) {  // (zeros past n, a multiple of 8, and past nb)
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        const int k = k0 + 32 * s + 8 * g;
+        const bool in = k < n;
+#pragma unroll
+        for (int t = 0; t < TR; t++) {
+          aw[s][t] = lm_u32x4{0u, 0u, 0u, 0u};
+          if (in) aw[s][t] = *reinterpret_cast<const lm_u32x4*>(wp[t] + k);
+        }
+#pragma unroll
+        for (int j = 0; j < TC; j++) {
+          const int b = (cb * CF + j) * 16 + m;
+          xa[s][j][0] = pz_f4u{0.0f, 0.0f, 0.0f, 0.0f};
+          xa[s][j][1] = xa[s][j][0];
+          if (in && b < nb) {
+            const float* xr = X + (size_t)b * ldx + k;
+            xa[s][j][0] = *reinterpret_cast<const pz_f4u*>(xr);
+            xa[s][j][1] = *reinterpret_cast<const pz_f4u*>(xr + 4);
+          }
+        }
+      }
+    };
+    fetch(0);
+    for (int k0 = 0; k0 < n; k0 += 32 * KS) {
+      lm_u32x4 h[KS][TC][3], a[KS][TR];
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+#pragma unroll
+        for (int j = 0; j < TC; j++) {
+          const pz_f4u u = xa[s][j][0], v = xa[s][j][1];
+          const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+          lm_split8(x, h[s][j]);
+        }
+#pragma unroll
+        for (int t = 0; t < TR; t++) {
+          a[s][t] = aw[s][t];
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            wmax = __builtin_elementwise_max(
+                wmax, __builtin_bit_cast(lm_u16x2, a[s][t][q] & 0x7fff7fffu));
+        }
+      }
+      fetch(k0 + 32 * KS);
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+#pragma unroll
+        for (int p = 2; p >= 0; p--)
+#pragma unroll
+          for (int j = 0; j < TC; j++)
+#pragma unroll
+            for (int t = 0; t < TR; t++)
+              acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  __builtin_bit_cast(lm_bf16x8, a[s][t]), __builtin_bit_cast(lm_bf16x8, h[s][j][p]),
+                  acc[t][j], 0, 0, 0);
+    }
+  } else {
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)sh;
+    const uint16_t* wbase = W + (size_t)row0 * n;
+    const int nst = (n + 32 * KS - 1) / (32 * KS);
+    // this wave's loads of W: row and 16-byte piece per lane.  Rows past V read
+    // row V - 1 (values unused); pieces past n read the row's last piece, which
+    // meets zero parts (and is non-finite only in a row flagged anyway).
+    uint32_t woff[WPW];
+    const int piece = KS == 1 ? g : (lane & 7) ^ (lane >> 3);
+#pragma unroll
+    for (int i = 0; i < WPW; i++) {
+      const int q = w * WPW + i;
+      const int r = KS == 1 ? q * 16 + m : q * 8 + (lane >> 3);
+      const int last = V - 1 - row0;
+      woff[i] = ((uint32_t)(r < last ? r : last) * (uint32_t)n + 8u * piece) * 2u;
+    }
+    const int klast = (nst - 1) * 32 * KS + 8 * piece;
+    const uint32_t wadj = klast < n ? 0u : (uint32_t)(klast - (n - 8)) * 2u;
+    const uint32_t xoff = (uint32_t)lane * 16u;
+    auto issue = [&](int c, int buf, int i) {  // load i of stage c into ring slot buf
+      const uint32_t l0 = lds0 + (uint32_t)buf * STG * 2;
+      if (i < WPW) {
+        const uint32_t off = woff[i] - (c == nst - 1 ? wadj : 0u), to = l0 + (w * WPW + i) * 1024;
+        lm_lds_load16<NT>(wbase + c * 32 * KS, off, to);
+      } else {
+        int q = w * XPW + i - WPW;
+        if (XF % NW) q = q < XF ? q : XF - 1;  // (the same bytes to the same place again)
+        const int s = q / (CF * 3), e = q - s * CF * 3;
+        lm_lds_load16<false>(xp + (((size_t)(c * KS + s) * ctt + cb * CF) * 3 + e) * LMX_FRAG, xoff,
+                      l0 + (WI + q) * 1024);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < NS - 1; i++)
+#pragma unroll
+      for (int q = 0; q < PER; q++) issue(i < nst ? i : nst - 1, i, q);
+    int buf = 0, nbuf = NS - 1;
+#pragma clang loop unroll(disable)
+    for (int c = 0; c < nst; c++) {
+      // stage c has arrived (the NS - 2 after it may be on their way), in every
+      // wave; and every wave is done reading the slot that is filled next
+      lm_wait<(NS - 2) * PER>();
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const uint16_t* sw = sh + buf * STG;
+      const uint16_t* sx = sw + WI * LMX_FRAG;
+      const int cn = c + NS - 1 < nst ? c + NS - 1 : nst - 1;  // (past the end: reloaded, unused)
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        lm_bf16x8 a[TR], b[3][TC];
+        const uint16_t* sxs = sx + (s * CF + wc * TC) * 3 * LMX_FRAG + lane * 8;
+#pragma unroll
+        for (int j = 0; j < TC; j++)
+          b[2][j] = *reinterpret_cast<const lm_bf16x8*>(sxs + (j * 3 + 2) * LMX_FRAG);
+#pragma unroll
+        for (int t = 0; t < TR; t++)
+          a[t] = *reinterpret_cast<const lm_bf16x8*>(
+              KS == 1 ? sw + (wr * TR + t) * LMX_FRAG + lane * 8
+                      : sw + (wr * TR + t) * 2 * LMX_FRAG + m * 64 + ((s * 4 + g) ^ (m & 7)) * 8);
+#pragma unroll
+        for (int p = 1; p >= 0; p--)
+#pragma unroll
+          for (int j = 0; j < TC; j++)
+            b[p][j] = *reinterpret_cast<const lm_bf16x8*>(sxs + (j * 3 + p) * LMX_FRAG);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int p = 2; p >= 0; p--)
+#pragma unroll
+          for (int j = 0; j < TC; j++)
+#pragma unroll
+            for (int t = 0; t < TR; t++) {
+              acc[t][j] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[p][j], acc[t][j], 0, 0, 0);
+              // the next stage's loads, one every few MFMAs of the first k-step
+              constexpr int SP = 3 * TR * TC / PER >= 4 ? 4 : 3 * TR * TC / PER;
+              static_assert(SP >= 1, "");
+              const int q = ((2 - p) * TC + j) * TR + t;
+              if (s == 0 && q % SP == SP - 1 && q / SP < PER) {
+                issue(cn, nbuf, q / SP);
+                __builtin_amdgcn_sched_barrier(0);
+              }
+            }
+#pragma unroll
+        for (int t = 0; t < TR; t++)
+          if (WC == 1 || t % WC == wc % TR) {
+            const lm_u32x4 q = __builtin_bit_cast(lm_u32x4, a[t]);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+              wmax = __builtin_elementwise_max(wmax,
+                                               __builtin_bit_cast(lm_u16x2, q[e] & 0x7fff7fffu));
+          }
+      }
+      asm volatile("" ::: "memory");
+      buf = buf + 1 == NS ? 0 : buf + 1;
+      nbuf = nbuf + 1 == NS ? 0 : nbuf + 1;
+    }
+    lm_wait<0>();
   }
-  lm_wait<0>();
   __syncthreads();  // the ring is free
   // an infinite or NaN weight anywhere in the workgroup's rows: those rows
   // again with fp32 fused multiply-adds over k (lanes), into the lanes that
@@ -553,18 +635,24 @@ template <int WR, int WC, int TR, int TC, int KS, int NS, int MODE>
 int launch_mfma(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* x, long ldx,
                 int nb, float* out, long ld, unsigned long long* keys, uint8_t* nan0) {
   constexpr int rows = WR * TR * 16, cols = WC * TC * 16;
-  const int ncb = (nb + cols - 1) / cols, nrt = (V + rows - 1) / rows, ctt = ncb * cols / 16;
-  const int ksteps = (n + 63) / 64 * 2;
-  hipLaunchKernelGGL(k_lmx_split, dim3(ksteps, ctt), dim3(64), 0, s->stream, x, ldx, nb, n, ctt,
-                     s->d_lmh_x);
-  PZ_HIP(s, hipGetLastError());
-  // (the 256-row tile is bound by the matrix cores: plain loads)
-  auto k = lm_once(V, n) && cols <= 128
-               ? k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE, (cols <= 128)>
-               : k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE, false>;
-  hipLaunchKernelGGL(k, dim3((unsigned)((nrt + 7) / 8 * 8) * ncb), dim3(64 * WR * WC), 0, s->stream,
-                     d_w, V, n, s->d_lmh_x, ctt, ncb, nrt, x, ldx, nb, out, ld, keys,
-                     s->max_batch, nan0);
+  const int ncb = (nb + cols - 1) / cols, nrt = (V + rows - 1) / rows;
+  const unsigned grid = (unsigned)((nrt + 7) / 8 * 8) * ncb;
+  if constexpr (NS == 0) {
+    hipLaunchKernelGGL((k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE, false>), dim3(grid),
+                       dim3(64 * WR * WC), 0, s->stream, d_w, V, n, nullptr, 0, ncb, nrt, x, ldx,
+                       nb, out, ld, keys, s->max_batch, nan0);
+  } else {
+    const int ctt = ncb * cols / 16, ksteps = (n + 63) / 64 * 2;
+    hipLaunchKernelGGL(k_lmx_split, dim3(ksteps, ctt), dim3(64), 0, s->stream, x, ldx, nb, n, ctt,
+                       s->d_lmh_x);
+    PZ_HIP(s, hipGetLastError());
+    // (the 256-row tile is bound by the matrix cores: plain loads)
+    auto k = lm_once(V, n) && cols <= 128
+                 ? k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE, (cols <= 128)>
+                 : k_lmhead_mfma<WR, WC, TR, TC, KS, NS, MODE, false>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(64 * WR * WC), 0, s->stream, d_w, V, n, s->d_lmh_x,
+                       ctt, ncb, nrt, x, ldx, nb, out, ld, keys, s->max_batch, nan0);
+  }
   PZ_HIP(s, hipGetLastError());
   return PZ_OK;
 }
@@ -608,21 +696,6 @@ int launch_tile(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* x
   return PZ_OK;
 }
 
-// The parts' workspace holds n weights of at least 16 batch rows: sized at
-// creation for PZ_LMX_ROWS rows of n = 8192 (or 16 rows of n = 131072); only
-// a longer row grows it.
-int lmx_reserve(pz_sampler* s, int n) {
-  const size_t need = (size_t)((n + 63) / 64) * 64 * 3 * 16;
-  if (need <= s->lmh_x_elems) return PZ_OK;
-  PZ_HIP(s, hipStreamSynchronize(s->stream));  // earlier calls may still read the old one
-  (void)hipFree(s->d_lmh_x);
-  s->d_lmh_x = nullptr;
-  s->lmh_x_elems = 0;
-  PZ_HIP(s, hipMalloc((void**)&s->d_lmh_x, need * sizeof(uint16_t)));
-  s->lmh_x_elems = need;
-  return PZ_OK;
-}
-
 // Batch tile: the smallest of 1, 2, 4, 8 that holds B rows (so three rows are
 // one read of W, not two), or the largest whose x tile fits the LDS budget
 // (0: n too large even for one row).
@@ -637,11 +710,14 @@ int run(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* d_x, int 
         float* d_logits, long ld) {
   // batch 4 and up: the matrix cores, W 16-byte aligned with rows of a
   // multiple of 8 weights; as many batch rows at a time as the parts'
-  // workspace holds, at most PZ_LMX_ROWS
+  // workspace holds (PZ_LMX_ROWS rows of n = 8192, 16 of n = 131072), at most
+  // PZ_LMX_ROWS; longer rows without it, since a call that only queues work
+  // neither allocates nor waits
   if (B >= 4 && n % 8 == 0 && ((uintptr_t)d_w & 15) == 0) {
-    const int rc = lmx_reserve(s, n);
-    if (rc != PZ_OK) return rc;
     const size_t fit = s->lmh_x_elems / ((size_t)((n + 63) / 64) * 64 * 3) / 16 * 16;
+    if (fit == 0)
+      return launch_mfma<4, 1, 4, 1, 2, 0, MODE>(s, d_w, V, n, d_x, ldx, B, d_logits, ld,
+                                                 s->d_lmh_keys, s->d_lmh_nan);
     const int most = fit < (size_t)PZ_LMX_ROWS ? (int)fit : PZ_LMX_ROWS;
     for (int b0 = 0; b0 < B; b0 += most) {
       const int nb = B - b0 < most ? B - b0 : most;

@@ -226,3 +226,42 @@ def test_equal_rows_give_equal_logits(torch_cuda, n):
             want = first[np.arange(B) % 7][:, np.arange(V) % period]
             assert (bits == want).all(), (B, np.argwhere(bits != want)[:3])
             assert (ids < period).all() and (gids == ids).all()
+
+
+@pytest.mark.parametrize("B", [4, 37])
+def test_rows_past_the_parts_workspace(torch_cuda, B):
+    """Rows of W longer than the workspace of the activations' parts serves
+    (131072 weights): the call queues its launches and nothing else -- no
+    device memory is taken -- and the sums are the ones of shorter rows, so
+    eight more zero weights change no bit."""
+    torch = torch_cuda
+    V, n = 300, 131072
+    print(f"case lmhead long rows B={B}", flush=True)
+    rng = np.random.default_rng(B)
+    w = rng.standard_normal((V, n), dtype=np.float32) * 0.02
+    x = rng.standard_normal((B, n), dtype=np.float32)
+    wb = bf16_bits(w)
+    longer = np.concatenate([wb, np.zeros((V, 8), np.uint16)], axis=1)
+    xl = np.concatenate([x, rng.standard_normal((B, 8), dtype=np.float32)], axis=1)
+    with pz.Sampler(64, V) as s:
+        logits, ids, gids = run(torch, wb, x, s)
+        check(f"long{B}", longer, xl, *run(torch, longer, xl, s))
+        got = run(torch, longer, xl, s)
+        assert (got[0].view(np.int32) == logits.view(np.int32)).all()
+        assert (got[1] == ids).all()
+        longer[V // 2, n + 7] = 0x7F80
+        got = run(torch, longer, xl, s)[0]
+        assert (got[:, V // 2] == np.copysign(np.inf, xl[:, n + 7])).all()
+    # twice the length: nothing is allocated (the first call loads the kernels)
+    d_w = torch.zeros((16, 2 * n + 8), dtype=torch.int16, device="cuda")
+    d_x = torch.ones((B, 2 * n + 8), dtype=torch.float32, device="cuda")
+    d_l = torch.empty((B, 16), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    with pz.Sampler(64, V) as s:
+        s.lm_head(d_w.data_ptr(), 16, n, d_x, B, n, d_l, 16)
+        s.sync()
+        free = torch.cuda.mem_get_info()[0]
+        s.lm_head(d_w.data_ptr(), 16, 2 * n + 8, d_x, B, 2 * n + 8, d_l, 16)
+        s.sync()
+        assert torch.cuda.mem_get_info()[0] == free
+    assert (d_l == 0).all()
