@@ -278,21 +278,24 @@ __global__ __launch_bounds__(64) void k_lmx_split(const float* __restrict__ X, l
 // 16 bytes per lane from base + off to LDS at byte address lds + 16 lane.
 // (Written as asm because for the builtin the compiler orders every later
 // LDS read of the workgroup behind all such loads; the stage loop below
-// waits for exactly the loads that it needs.  M0, the LDS base, is written
-// by whatever uses it, right before its use.)
+// waits for exactly the loads that it needs.  M0, the LDS base, is a clobber:
+// a value that the compiler keeps there is not taken for one that survived.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // (M0 is a reserved register)
 template <bool NT>
 __device__ __forceinline__ void lm_lds_load16(const void* base, uint32_t off, uint32_t lds) {
   if (NT)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
                  :
                  : "s"(lds), "v"(off), "s"(base)
-                 : "memory");
+                 : "m0", "memory");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :
                  : "s"(lds), "v"(off), "s"(base)
-                 : "memory");
+                 : "m0", "memory");
 }
+#pragma clang diagnostic pop
 // At most N of this wave's vector memory operations, and none of its LDS
 // operations, still outstanding.
 template <int N>
