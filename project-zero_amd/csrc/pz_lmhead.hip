@@ -208,10 +208,13 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
 //     XOR with the row in the source address so that the fragment reads do
 //     not meet in the banks.  The 256 x 256 tile's stage only fits with
 //     KS = 1; it is bound by the matrix cores, not by that.
-//   * NS = 0: no workspace, ring or stages -- a wave reads its tiles of W and
-//     splits its batch rows' activations in registers, KS k-steps ahead -- for
-//     rows longer than the workspace serves (16 batch rows at 4000 x 131080:
-//     3.2 ms, 3.7 where every workgroup staged the parts in LDS).
+//   * NS = 0: no workspace and no ring -- every workgroup makes its batch
+//     rows' parts itself, KS k-steps at a time, W straight into registers --
+//     for rows longer than the workspace serves (16 batch rows at 4000 x
+//     131080: 2.7 ms, 3.7 before there was a workspace) and for short ones
+//     (lm_own_parts).  KS = 2 leaves room for several workgroups per CU, which
+//     cover each other's waits: KS = 4 took 29.4 us where 2 takes 25.1 (32 x
+//     512 x 128256).
 //   * 128256 x 2560: 16 batch rows 112 us, 32 124, 64 167, 128 237, 256 405
 //     (one launch per 32 rows that split the activations in every workgroup
 //     took 143, 152, 301, 601 and 1203).
@@ -304,7 +307,7 @@ __device__ __forceinline__ void lm_wait() {
 }
 
 template <int WR, int WC, int TR, int TC, int KS, int NS, int MODE, bool NT>
-__global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(2, 8))) void
+__global__ __launch_bounds__(64 * WR * WC) __attribute__((amdgpu_waves_per_eu(NS ? 2 : 4, 8))) void
 k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __restrict__ xp,
               int ctt, int ncb, int nrt, const float* __restrict__ X, long ldx, int nb,
               float* __restrict__ logits, long ld, unsigned long long* __restrict__ keys,
@@ -314,9 +317,9 @@ k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __re
   constexpr int WI = RF * KS, XF = CF * 3 * KS;  // 1 KiB loads of a stage: weights, parts
   constexpr int WPW = WI / NW, XPW = (XF + NW - 1) / NW, PER = WPW + XPW;  // of a wave
   constexpr int STG = (WI + XF) * LMX_FRAG;
-  static_assert(WI % NW == 0 && (KS == 1 || KS == 2) && (NS == 0 || NS >= 2), "");
+  static_assert(NS == 0 || (WI % NW == 0 && (KS == 1 || KS == 2) && NS >= 2), "");
   static_assert(TR % WC == 0 || WC % TR == 0, "");
-  constexpr int SH = NS ? NS * STG : NW * CF * 64;
+  constexpr int SH = NS ? NS * STG : XF * LMX_FRAG;
   static_assert((size_t)SH * 2 >= NW * CF * 16 * 8, "the epilogue's keys reuse the ring");
   __shared__ __align__(16) uint16_t sh[SH];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -337,72 +340,86 @@ k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __re
   // their tiles in turn
   lm_u16x2 wmax = {0, 0};
   if constexpr (NS == 0) {
-    // no ring: a wave's own loads, KS k-steps ahead, its batch rows' parts
-    // made in registers
-    static_assert(NS > 0 || WC == 1, "");
+    // no workspace: the workgroup makes its batch rows' parts itself, KS
+    // k-steps at a time (in LDS as fragments, one per wave), W straight into
+    // registers
+    static_assert(NS > 0 || (WC == 1 && KS * CF <= NW), "");
+    constexpr int KC = 32 * KS;
     const uint16_t* wp[TR];
 #pragma unroll
     for (int t = 0; t < TR; t++) {
       const int r = row0 + (wr * TR + t) * 16 + m;
       wp[t] = W + (size_t)(r < V ? r : V - 1) * n;  // rows past V: a valid row, result unused
     }
-    lm_u32x4 aw[KS][TR];
-    pz_f4u xa[KS][TC][2];
-    auto fetch = [&](int k0) {  // (zeros past n, a multiple of 8, and past nb)
+    const int xb = (cb * CF + w % CF) * 16 + m, xk = (w / CF) * 32 + 8 * g;
+    float xv[8];
+    auto xload = [&](int k0) {  // (zeros past n, a multiple of 8, and past nb)
 #pragma unroll
-      for (int s = 0; s < KS; s++) {
-        const int k = k0 + 32 * s + 8 * g;
-        const bool in = k < n;
+      for (int e = 0; e < 8; e++) xv[e] = 0.0f;
+      if (w < KS * CF && xb < nb && k0 + xk < n) {
+        const float* xr = X + (size_t)xb * ldx + k0 + xk;
+        const pz_f4u u = *reinterpret_cast<const pz_f4u*>(xr);
+        const pz_f4u v = *reinterpret_cast<const pz_f4u*>(xr + 4);
 #pragma unroll
-        for (int t = 0; t < TR; t++) {
-          aw[s][t] = lm_u32x4{0u, 0u, 0u, 0u};
-          if (in) aw[s][t] = *reinterpret_cast<const lm_u32x4*>(wp[t] + k);
-        }
-#pragma unroll
-        for (int j = 0; j < TC; j++) {
-          const int b = (cb * CF + j) * 16 + m;
-          xa[s][j][0] = pz_f4u{0.0f, 0.0f, 0.0f, 0.0f};
-          xa[s][j][1] = xa[s][j][0];
-          if (in && b < nb) {
-            const float* xr = X + (size_t)b * ldx + k;
-            xa[s][j][0] = *reinterpret_cast<const pz_f4u*>(xr);
-            xa[s][j][1] = *reinterpret_cast<const pz_f4u*>(xr + 4);
-          }
+        for (int e = 0; e < 4; e++) {
+          xv[e] = u[e];
+          xv[e + 4] = v[e];
         }
       }
     };
-    fetch(0);
-    for (int k0 = 0; k0 < n; k0 += 32 * KS) {
-      lm_u32x4 h[KS][TC][3], a[KS][TR];
+    auto xstore = [&]() {
+      if (w >= KS * CF) return;
+      lm_u32x4 h[3];
+      lm_split8(xv, h);
 #pragma unroll
-      for (int s = 0; s < KS; s++) {
+      for (int p = 0; p < 3; p++)
+        *reinterpret_cast<lm_u32x4*>(sh + (w * 3 + p) * LMX_FRAG + lane * 8) = h[p];
+    };
+    auto wload = [&](lm_u32x4 (&a)[TR][KS], int k0) {
 #pragma unroll
-        for (int j = 0; j < TC; j++) {
-          const pz_f4u u = xa[s][j][0], v = xa[s][j][1];
-          const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
-          lm_split8(x, h[s][j]);
+      for (int t = 0; t < TR; t++)
+#pragma unroll
+        for (int q = 0; q < KS; q++) {
+          const int k = k0 + 32 * q + 8 * g;
+          a[t][q] = lm_u32x4{0u, 0u, 0u, 0u};
+          if (k < n) a[t][q] = *reinterpret_cast<const lm_u32x4*>(wp[t] + k);
         }
+    };
+    auto mma = [&](const lm_u32x4 (&a)[TR][KS]) {
+#pragma unroll
+      for (int q = 0; q < KS; q++) {
+        lm_bf16x8 b[3][TC];
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+#pragma unroll
+          for (int j = 0; j < TC; j++)
+            b[p][j] = *reinterpret_cast<const lm_bf16x8*>(
+                sh + ((q * CF + j) * 3 + p) * LMX_FRAG + lane * 8);
 #pragma unroll
         for (int t = 0; t < TR; t++) {
-          a[s][t] = aw[s][t];
 #pragma unroll
-          for (int q = 0; q < 4; q++)
+          for (int e = 0; e < 4; e++)
             wmax = __builtin_elementwise_max(
-                wmax, __builtin_bit_cast(lm_u16x2, a[s][t][q] & 0x7fff7fffu));
-        }
-      }
-      fetch(k0 + 32 * KS);
-#pragma unroll
-      for (int s = 0; s < KS; s++)
-#pragma unroll
-        for (int p = 2; p >= 0; p--)
+                wmax, __builtin_bit_cast(lm_u16x2, a[t][q][e] & 0x7fff7fffu));
 #pragma unroll
           for (int j = 0; j < TC; j++)
 #pragma unroll
-            for (int t = 0; t < TR; t++)
+            for (int p = 2; p >= 0; p--)
               acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  __builtin_bit_cast(lm_bf16x8, a[s][t]), __builtin_bit_cast(lm_bf16x8, h[s][j][p]),
-                  acc[t][j], 0, 0, 0);
+                  __builtin_bit_cast(lm_bf16x8, a[t][q]), b[p][j], acc[t][j], 0, 0, 0);
+        }
+      }
+    };
+    // every load of a chunk in flight at once; several workgroups per CU
+    // cover the waits
+    for (int k0 = 0; k0 < n; k0 += KC) {
+      lm_u32x4 a[TR][KS];
+      xload(k0);
+      wload(a, k0);
+      __syncthreads();  // the chunk before is done with the LDS
+      xstore();
+      __syncthreads();
+      mma(a);
     }
   } else {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)sh;
@@ -634,6 +651,21 @@ int lm_tile_for(int V, int nb, int most, int n_cu) {
   return best;
 }
 
+// Batches of 4 to 32 whose workgroups make the parts themselves: where the
+// launch that makes them once takes longer than it saves.  One round of
+// 256-row workgroups: rows of up to 256 (us, own / once, as the kernel that
+// staged the parts in every workgroup before: 4 x 128 x 8000 5.4 / 7.9, 5.6;
+// 32 x 256 x 50257 12.5 / 13.4, 13.7; but 32 x 512 x 50257 18.3 / 17.2, 21.5).
+// More rounds, where a ring per workgroup also fills and drains too often: up
+// to 1024, past the Infinity Cache 768 (32 x 256 x 128256 15.6 / 20.7, 20.9;
+// fused 32 x 1024 x 128256 44.0 / 48.3, 46.1; 16 x 768 x 200000 68.7 / 74.9,
+// 75.0; but 32 x 1024 x 200000 107.7 / 99.3, 109.6).
+bool lm_own_parts(int V, int n, int B, int n_cu) {
+  if (B > 32) return false;
+  if (V <= 256 * n_cu) return n <= 256;
+  return n <= (lm_once(V, n) ? 768 : 1024);
+}
+
 template <int WR, int WC, int TR, int TC, int KS, int NS, int MODE>
 int launch_mfma(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* x, long ldx,
                 int nb, float* out, long ld, unsigned long long* keys, uint8_t* nan0) {
@@ -718,9 +750,11 @@ int run(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* d_x, int 
   // neither allocates nor waits
   if (B >= 4 && n % 8 == 0 && ((uintptr_t)d_w & 15) == 0) {
     const size_t fit = s->lmh_x_elems / ((size_t)((n + 63) / 64) * 64 * 3) / 16 * 16;
-    if (fit == 0)
-      return launch_mfma<4, 1, 4, 1, 2, 0, MODE>(s, d_w, V, n, d_x, ldx, B, d_logits, ld,
-                                                 s->d_lmh_keys, s->d_lmh_nan);
+    if (fit == 0 || lm_own_parts(V, n, B, s->n_cu))
+      return B <= 16 ? launch_mfma<8, 1, 2, 1, 2, 0, MODE>(s, d_w, V, n, d_x, ldx, B, d_logits, ld,
+                                                           s->d_lmh_keys, s->d_lmh_nan)
+                     : launch_mfma<8, 1, 2, 2, 2, 0, MODE>(s, d_w, V, n, d_x, ldx, B, d_logits, ld,
+                                                           s->d_lmh_keys, s->d_lmh_nan);
     const int most = fit < (size_t)PZ_LMX_ROWS ? (int)fit : PZ_LMX_ROWS;
     for (int b0 = 0; b0 < B; b0 += most) {
       const int nb = B - b0 < most ? B - b0 : most;

@@ -160,7 +160,8 @@ def test_fused_argmax_ties_and_nan(torch_cuda):
 @pytest.mark.parametrize("B,V,n", [
     (4, 1, 8), (16, 129, 40), (17, 255, 96), (32, 4099, 1048), (33, 257, 72), (64, 512, 2560),
     (65, 1000, 104), (128, 4099, 2056), (129, 300, 32), (256, 4099, 264), (257, 513, 160),
-    (530, 1025, 64), (9, 1025, 2048), (40, 800, 4096), (20, 40000, 136), (100, 70001, 72), (200, 70001, 24), (90, 700, 24576)])
+    (530, 1025, 64), (9, 1025, 2048), (40, 800, 4096), (20, 40000, 136), (100, 70001, 72), (200, 70001, 24), (90, 700, 24576),
+    (5, 66000, 328), (16, 66000, 40), (32, 66001, 72), (17, 300, 248)])
 def test_lm_head_matrix_core_tiles(torch_cuda, B, V, n):
     """Every tile shape of the GEMM, unfused against float64 and fused against
     the argmax of the unfused logits; row V // 2 holds an infinite weight (its
@@ -202,8 +203,9 @@ def test_lm_head_matrix_core_tiles(torch_cuda, B, V, n):
 
 
 # row lengths around the multiples of 2048 (rows of W a multiple of 4 KiB
-# apart), batches in every tile of the GEMM and in more than one chunk
-@pytest.mark.parametrize("n", [2048, 2056, 2560, 4096, 6144])
+# apart) and short ones with and without the workspace, batches in every tile
+# of the GEMM and in more than one chunk
+@pytest.mark.parametrize("n", [64, 72, 256, 264, 2048, 2056, 2560, 4096, 6144])
 def test_equal_rows_give_equal_logits(torch_cuda, n):
     """From four batch rows on, a logit depends on its row of W and its
     activations alone: not on where the row lies in the vocabulary, on the
