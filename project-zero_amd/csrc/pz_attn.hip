@@ -473,11 +473,14 @@ extern "C" int pz_attn_softmax(pz_sampler* s, const float* d_in, long ld_in, flo
     if (rc != -2) return fail(s, PZ_EDEVICE, "attention softmax launch failed");
   }
   // a workgroup per row runs one row per CU at a time, a wave per row all of
-  // them: beyond a round or two of workgroups the waves are quicker (us,
-  // workgroups / waves: n = 2048, 256 rows 14 / 19, 512 25 / 19, 2048 89 /
-  // 23; n = 4096, 512 rows 29 / 32, 1024 53 / 35, 2048 103 / 42)
-  const int cus = s->n_cu > 0 ? s->n_cu : 256;
-  const bool waves = n <= ATTN_WAVE_MAX && n_rows > (n <= 2048 ? cus : 2 * cus);
+  // them: beyond a round or two of workgroups the waves are quicker (us, rows
+  // of full length and ragged ones, workgroups / waves: n = 2048, 257 rows 29
+  // / 31 and 25 / 30, 288 rows 32 / 31 and 31 / 29, 2048 rows 99 / 35 and 89 /
+  // 32; n = 4096, 513 rows 43 / 46 and 37 / 43, 576 rows 50 / 45 and 43 / 43,
+  // 2048 rows 115 / 54 and 101 / 47)
+  const long cus = s->n_cu > 0 ? s->n_cu : 256;
+  const bool waves =
+      n <= ATTN_WAVE_MAX && (n <= 2048 ? 8 * (long)n_rows >= 9 * cus : 4 * (long)n_rows >= 9 * cus);
   if (n > ATTN_WAVE_SHORT && n <= ATTN_ROW_MAX && !waves) {
     const int rc = launch_row(s, d_in, ld_in, d_out, ld_out, n_rows, n, d_len);
     if (rc == 0) return PZ_OK;

@@ -126,7 +126,9 @@ def test_special_values(torch_cuda, n):
 
 
 @pytest.mark.parametrize("rows,n", [(256, 1025), (257, 1025), (300, 2048), (257, 2049),
-                                    (513, 2049), (515, 4095), (520, 4096), (600, 4097)])
+                                    (513, 2049), (515, 4095), (520, 4096), (600, 4097),
+                                    (287, 2048), (288, 1025), (575, 2049), (576, 2049),
+                                    (577, 4096)])
 def test_many_rows(torch_cuda, rows, n):
     """Around the row counts from which rows of up to 4096 scores take a wave
     each instead of a workgroup, over ragged lengths, with rows whose sums
