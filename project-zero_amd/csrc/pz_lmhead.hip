@@ -77,7 +77,6 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
     float* __restrict__ logits, long ld, unsigned long long* __restrict__ keys,
     uint8_t* __restrict__ nan0) {
   extern __shared__ __align__(16) float xs[];  // [BT][n rounded up to 512]
-  __shared__ unsigned long long best_sh[LM_WAVES][BT];
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nchunk = (n + 511) >> 9;
@@ -164,13 +163,19 @@ __global__ __launch_bounds__(64 * LM_WAVES) void k_lmhead(
     }
   }
   if (MODE == 1) {
+    // the waves' keys meet where the activations were: LDS of their own would
+    // leave room for one workgroup per CU less where the activations take a
+    // half or a quarter of it (8 batch rows of 2049 weights x 50257: 370 us
+    // with it, 238 without; 4 of 5001 x 32000: 412 and 277)
+    unsigned long long* best_sh = reinterpret_cast<unsigned long long*>(xs);  // [LM_WAVES][BT]
+    __syncthreads();
     if (lane == 0)
 #pragma unroll
-      for (int b = 0; b < BT; b++) best_sh[w][b] = best[b];
+      for (int b = 0; b < BT; b++) best_sh[w * BT + b] = best[b];
     __syncthreads();
     if (tid < BT && tid < nb) {
-      unsigned long long m = best_sh[0][tid];
-      for (int i = 1; i < LM_WAVES; i++) m = best_sh[i][tid] > m ? best_sh[i][tid] : m;
+      unsigned long long m = best_sh[tid];
+      for (int i = 1; i < LM_WAVES; i++) m = best_sh[i * BT + tid] > m ? best_sh[i * BT + tid] : m;
       if (m) atomicMax(&keys[tid], m);
     }
   }
