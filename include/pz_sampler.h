@@ -75,7 +75,13 @@ typedef struct {
 } pz_row_params;
 
 /* Creates a sampler on `device` for batches of up to max_batch rows of up to
- * max_vocab logits and histories of up to max_hist ids (max_hist <= 2048). */
+ * max_vocab logits and histories of up to max_hist ids (max_hist <= 2048).
+ * Allocates all its device memory but the workspaces of verification and of
+ * long attention rows, which their first calls allocate.  The largest part is
+ * the scratch that sorts top-p rows with wide nuclei: 16 bytes per id (ids
+ * rounded up to a power of two, at most 262144) for each row sorted at once,
+ * which is min(max_batch, compute units) rows while that is at most a 64th of
+ * the free device memory (512 MiB for 256 rows of 128256 ids), else fewer. */
 PZ_API int pz_sampler_create(pz_sampler **out, int max_batch, int max_vocab,
                       int max_hist, int device);
 PZ_API void pz_sampler_destroy(pz_sampler *s);

@@ -10,12 +10,14 @@
 #include "pz_split.h"
 
 // Device scratch owned by a sampler (carved from one allocation).
-// Rows the top-p fallback kernel sorts at once: one per CU, as its LDS has it
-// (2 MiB of scratch each at 128256 ids, at most max_batch of them).  With 32,
-// 256 rows of 128256 ids at temperature 1, top-p 0.95 -- most of them wider
-// than the gather -- took 5282 us, where 256 slots take 972; 100 such rows of
-// 200000 ids 5562 and 1726.
-constexpr int PZ_FB_SLOTS = 256;
+// Rows the top-p fallback kernel sorts at once: one per CU, as its LDS has it,
+// at most max_batch, while they take no more than a 64th of the device's free
+// memory (2 MiB each at 128256 ids, 4 above 131072: 512 MiB or 1 GiB for 256
+// rows); up to PZ_FB_SLOTS of them in any case, fewer where even those cannot
+// be allocated (pz_slots.h).  With 32, 256 rows of 128256 ids at temperature 1,
+// top-p 0.95 -- most of them wider than the gather -- took 5282 us, where 256
+// slots take 972; 100 such rows of 200000 ids 5562 and 1726.
+constexpr int PZ_FB_SLOTS = 32;
 constexpr int PZ_COUNTERS = 64;        // words of pz_scratch::counters
 constexpr int PZ_TOPP_MAX_V = 200000;  // top_p.c:27 (larger rows take argmax)
 constexpr int PZ_TOPP_CAPG = 12288;    // top-p candidates a row can gather for the LDS sort
@@ -28,7 +30,7 @@ struct pz_scratch {
   uint64_t* fb_keys;  // [fb_slots][slot_n] sort buffers of the fallback
   uint64_t* fb_keys2; // [fb_slots][slot_n] its second buffer (keys in bin order)
   int slot_n;         // power of two >= min(max_vocab, PZ_TOPP_MAX_V)
-  int fb_slots;       // min(PZ_FB_SLOTS, max_batch) sort slots
+  int fb_slots;       // sort slots (at least 1)
 };
 
 // Bytes of scratch for max_batch rows of up to max_vocab ids with at most

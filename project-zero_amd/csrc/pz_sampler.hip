@@ -18,6 +18,7 @@
 #include "pz_launch.h"
 #include "pz_params.h"
 #include "pz_sampler_impl.h"
+#include "pz_slots.h"
 
 namespace {
 
@@ -123,9 +124,22 @@ extern "C" int pz_sampler_create(pz_sampler** out, int max_batch, int max_vocab,
     return bail(PZ_EDEVICE);
   s->res_params = new (std::nothrow) pz_row_params_dev[B];
   if (!s->res_params) return bail(PZ_ENOMEM);
-  s->scratch_bytes = pz_scratch_layout(max_batch, max_vocab, PZ_FB_SLOTS, nullptr, nullptr);
-  if (hipMalloc(&s->d_scratch, s->scratch_bytes) != hipSuccess) return bail(PZ_ENOMEM);
-  pz_scratch_layout(max_batch, max_vocab, PZ_FB_SLOTS, s->d_scratch, &s->sc);
+  size_t free_bytes = 0, total_bytes = 0;
+  if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) return bail(PZ_EDEVICE);
+  auto scratch_bytes = [&](int slots) {
+    return pz_scratch_layout(max_batch, max_vocab, slots, nullptr, nullptr);
+  };
+  const int slots = pz_take_slots(
+      max_batch < s->n_cu ? max_batch : s->n_cu, PZ_FB_SLOTS, free_bytes, scratch_bytes,
+      [&](int n) {
+        s->scratch_bytes = scratch_bytes(n);
+        if (hipMalloc(&s->d_scratch, s->scratch_bytes) == hipSuccess) return true;
+        s->d_scratch = nullptr;
+        (void)hipGetLastError();  // (or the next launch's check would report it)
+        return false;
+      });
+  if (!slots) return bail(PZ_ENOMEM);
+  pz_scratch_layout(max_batch, max_vocab, slots, s->d_scratch, &s->sc);
   // queue counters start at zero; the fallback kernel re-zeroes them after
   // each launch that read them
   if (hipMemset(s->sc.counters, 0, PZ_COUNTERS * sizeof(int32_t)) != hipSuccess)
