@@ -38,6 +38,7 @@
 
 #include "../../include/pz_sampler.h"
 #include "pz_device.h"
+#include "pz_lmtile.h"
 #include "pz_sampler_impl.h"
 
 namespace {
@@ -63,11 +64,6 @@ __device__ __forceinline__ void widen8(const lm_u32x4 q, float (&w)[8]) {
 __device__ __forceinline__ uint64_t argmax_key(float v, int id) {
   return ((uint64_t)pz_key(v) << 32) | (uint64_t)(0xffffffffu - (uint32_t)id);
 }
-
-// Weights the Infinity Cache (256 MB) cannot hold from one call to the next
-// are loaded non-temporally: 128256 x 2560 at batch 1 114 -> 98 us, at 8
-// (matrix cores) 116 -> 107; 50257 x 1024, which it can hold, 18.2 -> 19.5.
-bool lm_once(int V, int n) { return (size_t)V * n * 2 > ((size_t)256 << 20); }
 
 // MODE 0: write logits.  MODE 1: argmax keys.  VEC: n % 8 == 0 and W 16-byte
 // aligned (one 16-byte load per 8 weights), else element loads.
@@ -625,52 +621,6 @@ k_lmhead_mfma(const uint16_t* __restrict__ W, int V, int n, const uint16_t* __re
   }
 }
 
-// One tile shape of the GEMM: its batch block, rows per workgroup, workgroups
-// per CU (LDS), k-steps per stage, and the time of one round of workgroups
-// on every CU at n = 2560 (us, measured at V = 128256).
-struct LmTile {
-  int cols, rows, per_cu;
-  float round_us;
-};
-constexpr LmTile LM_TILE_SHAPES[] = {
-    {256, 256, 1, 192.0f}, {128, 256, 1, 107.0f}, {64, 256, 1, 83.0f}, {32, 256, 1, 64.0f},
-    {32, 128, 2, 67.0f},   {16, 256, 1, 59.0f},   {16, 128, 2, 62.0f}};
-constexpr int LM_TILE_COUNT = sizeof(LM_TILE_SHAPES) / sizeof(LM_TILE_SHAPES[0]);
-
-// The shape with the least time for nb batch rows: rounds of workgroups times
-// a round's time.
-int lm_tile_for(int V, int nb, int most, int n_cu) {
-  int best = LM_TILE_COUNT - 1;
-  float best_us = __builtin_inff();
-  for (int i = 0; i < LM_TILE_COUNT; i++) {
-    const LmTile& t = LM_TILE_SHAPES[i];
-    if ((nb + t.cols - 1) / t.cols * t.cols > most) continue;  // parts past the workspace
-    const long wgs = (long)((V + t.rows - 1) / t.rows) * ((nb + t.cols - 1) / t.cols);
-    const long slots = (long)n_cu * t.per_cu;
-    const float us = (float)((wgs + slots - 1) / slots) * t.round_us;
-    if (us < best_us) {
-      best = i;
-      best_us = us;
-    }
-  }
-  return best;
-}
-
-// Batches of 4 to 32 whose workgroups make the parts themselves: where the
-// launch that makes them once takes longer than it saves.  One round of
-// 256-row workgroups: rows of up to 256 (us, own / once, as the kernel that
-// staged the parts in every workgroup before: 4 x 128 x 8000 5.4 / 7.9, 5.6;
-// 32 x 256 x 50257 12.5 / 13.4, 13.7; but 32 x 512 x 50257 18.3 / 17.2, 21.5).
-// More rounds, where a ring per workgroup also fills and drains too often: up
-// to 1024, past the Infinity Cache 768 (32 x 256 x 128256 15.6 / 20.7, 20.9;
-// fused 32 x 1024 x 128256 44.0 / 48.3, 46.1; 16 x 768 x 200000 68.7 / 74.9,
-// 75.0; but 32 x 1024 x 200000 107.7 / 99.3, 109.6).
-bool lm_own_parts(int V, int n, int B, int n_cu) {
-  if (B > 32) return false;
-  if (V <= 256 * n_cu) return n <= 256;
-  return n <= (lm_once(V, n) ? 768 : 1024);
-}
-
 template <int WR, int WC, int TR, int TC, int KS, int NS, int MODE>
 int launch_mfma(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* x, long ldx,
                 int nb, float* out, long ld, unsigned long long* keys, uint8_t* nan0) {
@@ -775,9 +725,7 @@ int run(pz_sampler* s, const uint16_t* d_w, int V, int n, const float* d_x, int 
         PZ_LM_CASE(1, 4, 2, 4, 4, 2, 2);
         PZ_LM_CASE(2, 4, 2, 4, 2, 2, 2);
         PZ_LM_CASE(3, 8, 1, 2, 2, 2, 3);
-        PZ_LM_CASE(4, 4, 1, 2, 2, 2, 2);
-        PZ_LM_CASE(5, 8, 1, 2, 1, 2, 4);
-        default: r = launch_mfma<4, 1, 2, 1, 2, 3, MODE>(s, d_w, V, n, x, ldx, nb, out, ld, keys, nan0);
+        default: r = launch_mfma<8, 1, 2, 1, 2, 4, MODE>(s, d_w, V, n, x, ldx, nb, out, ld, keys, nan0);
 #undef PZ_LM_CASE
       }
       if (r != PZ_OK) return r;

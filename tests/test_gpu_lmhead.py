@@ -154,18 +154,28 @@ def test_fused_argmax_ties_and_nan(torch_cuda):
     check("ties", wb, x, logits, ids, gids, check_logits=False)
 
 
-# the matrix-core tile shapes: batch blocks of 16 .. 256 and their edges, two
-# chunks of 256, row tiles of 128 and 256 and their edges, k below one step,
-# off a step and off a stage
-@pytest.mark.parametrize("B,V,n", [
+# edges of the matrix-core paths: batch blocks of 16 .. 256, two chunks of 256,
+# row tiles of 256, k below one step, off a step and off a stage, with and
+# without the workspace (tests/test_lmhead_tiles.py says which path each takes)
+TILE_CASES = [
     (4, 1, 8), (16, 129, 40), (17, 255, 96), (32, 4099, 1048), (33, 257, 72), (64, 512, 2560),
     (65, 1000, 104), (128, 4099, 2056), (129, 300, 32), (256, 4099, 264), (257, 513, 160),
-    (530, 1025, 64), (9, 1025, 2048), (40, 800, 4096), (20, 40000, 136), (100, 70001, 72), (200, 70001, 24), (90, 700, 24576),
-    (5, 66000, 328), (16, 66000, 40), (32, 66001, 72), (17, 300, 248)])
+    (530, 1025, 64), (9, 1025, 2048), (40, 800, 4096), (20, 40000, 136), (100, 70001, 72),
+    (200, 70001, 24), (90, 700, 24576), (5, 66000, 328), (16, 66000, 40), (32, 66001, 72),
+    (17, 300, 248)]
+# vocabularies for which the other tile shapes are chosen: the 256 x 256 tile
+# with an odd number of k-steps and an end off a step, the 64-row tile, and W
+# past the Infinity Cache in every tile that then loads it non-temporally
+LARGE_CASES = [
+    (200, 33000, 40), (256, 65003, 72), (229, 40001, 104), (48, 33000, 40), (64, 40001, 104),
+    (8, 131201, 1032), (20, 131201, 1032), (60, 131201, 1032), (100, 131201, 1032)]
+
+
+@pytest.mark.parametrize("B,V,n", TILE_CASES)
 def test_lm_head_matrix_core_tiles(torch_cuda, B, V, n):
-    """Every tile shape of the GEMM, unfused against float64 and fused against
-    the argmax of the unfused logits; row V // 2 holds an infinite weight (its
-    logits are +-inf by the sign of the activation it meets)."""
+    """The GEMM's edges, unfused against float64 and fused against the argmax of
+    the unfused logits; row V // 2 holds an infinite weight (its logits are
+    +-inf by the sign of the activation it meets)."""
     torch = torch_cuda
     print(f"case lmhead tiles B={B} V={V} n={n}", flush=True)
     rng = np.random.default_rng(B * 7 + n)
@@ -267,3 +277,45 @@ def test_rows_past_the_parts_workspace(torch_cuda, B):
         s.sync()
         assert torch.cuda.mem_get_info()[0] == free
     assert (d_l == 0).all()
+
+
+@pytest.mark.parametrize("B,V,n", LARGE_CASES)
+def test_lm_head_large_tiles(torch_cuda, B, V, n):
+    """The tile shapes of large vocabularies: W repeats 331 rows, one of them
+    with an infinite weight, so every logit is known from the first 331 (those
+    against float64); rows longer than their entries, off 16 bytes."""
+    torch = torch_cuda
+    print(f"case lmhead large tiles B={B} V={V} n={n}", flush=True)
+    rng = np.random.default_rng(B + n)
+    P, r = 331, 100
+    base = bf16_bits(rng.standard_normal((P, n), dtype=np.float32) * 0.02)
+    x = rng.standard_normal((B, n), dtype=np.float32)
+    finite = base.copy()
+    finite[r] = 0
+    base[r, n - 1] = 0x7F80
+    d_w = to_dev(torch, base.view(np.int16)).repeat(V // P + 1, 1)[:V].contiguous()
+    ld, ldx = V + 3, n + 5
+    d_x = torch.full((B, ldx), float("nan"), dtype=torch.float32, device="cuda")
+    d_x[:, :n] = to_dev(torch, x)
+    d_l = torch.full((B, ld), -7.0, dtype=torch.float32, device="cuda")
+    d_i = torch.full((B,), -9, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    with pz.Sampler(B, V) as s:
+        s.lm_head(d_w.data_ptr(), V, n, d_x, B, ldx, d_l, ld)
+        s.lm_head_argmax(d_w.data_ptr(), V, n, d_x, B, ldx, d_i)
+        s.sync()
+    logits = d_l.cpu().numpy()
+    ids = d_i.cpu().numpy()
+    first = logits[:, :P].copy()
+    assert (logits[:, :V].view(np.int32) == first.view(np.int32)[:, np.arange(V) % P]).all()
+    assert (logits[:, V:] == -7.0).all()
+    want = np.array([po.oracle().orc_argmax(
+        np.ascontiguousarray(q).ctypes.data_as(po._P), q.size) for q in first], np.int32)
+    assert (ids == want).all()
+    assert (first[:, r] == np.copysign(np.inf, x[:, n - 1])).all()
+    first[:, r] = 0.0
+    ex, bound = exact(finite, x)
+    err = np.abs(first.astype(np.float64) - ex)
+    tol = n * 2.0 ** -24 * bound + 1e-30
+    print(f"B{B} V{V} n{n}: max |err| / bound = {float((err / tol).max()):.4f}", flush=True)
+    assert (err <= tol).all()
