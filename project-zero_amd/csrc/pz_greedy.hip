@@ -20,12 +20,18 @@
 
 namespace {
 
-template <int BLOCK, int U, class F4>
-__device__ __forceinline__ void gr_load(const F4* x4, int n4, int base, pz_f4 (&v)[U]) {
+// VEC: 2 rows start 16-byte aligned, 1 at any address (pz_f4u; a template
+// argument would lose its alignment), 0 fewer than four ids.
+template <int BLOCK, int U, int VEC>
+__device__ __forceinline__ void gr_load(const float* x, int n4, int base, pz_f4 (&v)[U]) {
 #pragma unroll
   for (int u = 0; u < U; u++) {
     const int i4 = base + u * BLOCK + (int)threadIdx.x;
-    v[u] = __builtin_nontemporal_load(&x4[i4 < n4 ? i4 : n4 - 1]);  // unconditional
+    const float* p = x + 4 * (long)(i4 < n4 ? i4 : n4 - 1);  // unconditional
+    if (VEC == 1)
+      v[u] = __builtin_nontemporal_load(reinterpret_cast<const pz_f4u*>(p));
+    else
+      v[u] = __builtin_nontemporal_load(reinterpret_cast<const pz_f4*>(p));
   }
 }
 
@@ -95,18 +101,18 @@ __device__ __forceinline__ void gr_group(const PzPenalty& P, const pz_row_params
 // One exit only (the loop condition): a break in the middle of the loop body
 // makes the compiler merge paths on which the other set's loads are still
 // in flight, and it then drains every load at the loop head.
-template <int BLOCK, int U, bool TEMPER, bool PEN, class F4>
+template <int BLOCK, int U, int VEC, bool TEMPER, bool PEN>
 __device__ __forceinline__ void gr_stream(const PzPenalty& P, const pz_row_params_dev& prm,
-                                          int lo, const F4* x4, int n4, pz_f4 (&a)[U],
+                                          int lo, const float* x, int n4, pz_f4 (&a)[U],
                                           pz_f4 (&b)[U], GrBest& B) {
   constexpr int STEP = BLOCK * U;
   const int ng = (n4 + STEP - 1) / STEP;
   int g = 0;
   for (; g + 1 < ng; g += 2) {
-    gr_load<BLOCK, U>(x4, n4, (g + 1) * STEP, b);
+    gr_load<BLOCK, U, VEC>(x, n4, (g + 1) * STEP, b);
     gr_group<BLOCK, U, TEMPER, PEN>(P, prm, lo, n4, g * STEP, a, B);
     __builtin_amdgcn_sched_barrier(0);
-    gr_load<BLOCK, U>(x4, n4, (g + 2) * STEP, a);
+    gr_load<BLOCK, U, VEC>(x, n4, (g + 2) * STEP, a);
     gr_group<BLOCK, U, TEMPER, PEN>(P, prm, lo, n4, (g + 1) * STEP, b, B);
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -119,16 +125,6 @@ __device__ __forceinline__ void gr_stream(const PzPenalty& P, const pz_row_param
 // guard, which take the argmax of the tempered row (top_p.c:33-34, after
 // apply_temperature).  PEN: some row of the launch has an active penalty;
 // every row then builds the bitmap (all zero where the row has none).
-// VEC: 2 rows start 16-byte aligned, 1 at any address (pz_f4u), 0 fewer than
-// four ids.
-template <int VEC>
-struct GrF4 {
-  typedef pz_f4 type;
-};
-template <>
-struct GrF4<1> {
-  typedef pz_f4u type;
-};
 template <int BLOCK, int U, int VEC, bool TEMPER, bool PEN>
 __global__ __launch_bounds__(BLOCK) void k_greedy(
     const float* __restrict__ logits, long ld, int V,
@@ -144,8 +140,6 @@ __global__ __launch_bounds__(BLOCK) void k_greedy(
   const float* x = logits + (long)row * ld;
   const int32_t* hrow = hist ? hist + (long)row * H : nullptr;
   const int tid = threadIdx.x;
-  typedef typename GrF4<VEC>::type F4;
-  const F4* x4 = reinterpret_cast<const F4*>(x);
   const int n4 = VEC ? V >> 2 : 0;  // VEC launches have V >= 4, so n4 >= 1
 
   // Prologue ordered for the in-order load counter: the history id of one
@@ -155,7 +149,7 @@ __global__ __launch_bounds__(BLOCK) void k_greedy(
   int hid0 = -1;
   if (hrow && tid < H) hid0 = hrow[tid];
   pz_f4 a[U], b[U];
-  if (VEC) gr_load<BLOCK, U>(x4, n4, 0, a);  // unconditional within the launch
+  if (VEC) gr_load<BLOCK, U, VEC>(x, n4, 0, a);  // unconditional within the launch
   const float x0 = tid == 0 ? x[0] : 0.0f;
   __builtin_amdgcn_sched_barrier(0);
 
@@ -187,7 +181,7 @@ __global__ __launch_bounds__(BLOCK) void k_greedy(
     B.bv = -__builtin_inff();
     B.b4 = 0x7fffffff;
     B.bx = pz_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    gr_stream<BLOCK, U, TEMPER, PEN>(P, prm, 0, x4, n4, a, b, B);
+    gr_stream<BLOCK, U, VEC, TEMPER, PEN>(P, prm, 0, x, n4, a, b, B);
     if (B.b4 != 0x7fffffff) {  // the first of the float4's values equal to the best
       bv = B.bv;
       bi = (B.b4 << 2) + (B.bx.x == bv ? 0 : B.bx.y == bv ? 1 : B.bx.z == bv ? 2 : 3);
@@ -260,14 +254,13 @@ __global__ __launch_bounds__(BLOCK) void k_greedy_split(
   const float* x = logits + (long)row * ld;
   const int32_t* hrow = hist ? hist + (long)row * H : nullptr;
   const int tid = threadIdx.x;
-  typedef typename GrF4<VEC>::type F4;
-  const F4* x4 = reinterpret_cast<const F4*>(x + lo);
+  const float* xl = x + lo;
   const int n4 = (hi - lo) >> 2;  // 0 only for a last range of 1-3 ids
 
   int hid0 = -1;
   if (hrow && tid < H) hid0 = hrow[tid];
   pz_f4 a[U], b[U];
-  if (n4 > 0) gr_load<BLOCK, U>(x4, n4, 0, a);
+  if (n4 > 0) gr_load<BLOCK, U, VEC>(xl, n4, 0, a);
   const float x0 = (sl == 0 && tid == 0) ? x[0] : 0.0f;
   __builtin_amdgcn_sched_barrier(0);
 
@@ -299,7 +292,7 @@ __global__ __launch_bounds__(BLOCK) void k_greedy_split(
     B.bv = -__builtin_inff();
     B.b4 = 0x7fffffff;
     B.bx = pz_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    gr_stream<BLOCK, U, TEMPER, PEN>(P, prm, lo, x4, n4, a, b, B);
+    gr_stream<BLOCK, U, VEC, TEMPER, PEN>(P, prm, lo, xl, n4, a, b, B);
     if (B.b4 != 0x7fffffff) {
       bv = B.bv;
       bi = lo + (B.b4 << 2) + (B.bx.x == bv ? 0 : B.bx.y == bv ? 1 : B.bx.z == bv ? 2 : 3);
