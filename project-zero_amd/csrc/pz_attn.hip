@@ -188,7 +188,9 @@ int launch_wave(pz_sampler* s, const float* d_in, long ld_in, float* d_out, long
 // ---- one workgroup per row ----------------------------------------------------
 constexpr int AR_BLOCK = 1024;
 constexpr int AR_WAVES = AR_BLOCK / 64;
-constexpr int ATTN_ROW_MAX = 128 * 256;  // longest row of k_attn_row (128 segments)
+constexpr int AR_SEGS = 128;              // segments of k_attn_row's longest row
+constexpr int ATTN_ROW_MAX = AR_SEGS * 256;
+static_assert(pz_sp_walk_block_ok(AR_BLOCK), "");
 
 // Row r's scores as the walk reads them: V = the row's valid length.
 struct AttnRow {
@@ -203,7 +205,7 @@ struct AttnRow {
 };
 
 struct AttnShared {
-  float est[128];
+  float est[AR_SEGS];
   float red[AR_WAVES];
   uint32_t bad[AR_WAVES];
   float carry;
@@ -218,6 +220,7 @@ template <int NSW, bool VEC_IN>
 __global__ __launch_bounds__(AR_BLOCK) void k_attn_row(const float* in, long ld_in, float* out,
                                                       long ld_out, int n_rows, int n,
                                                       const int32_t* lens, int nc) {
+  static_assert(NSW * AR_WAVES <= AR_SEGS, "a segment's estimate per wave and turn");
   extern __shared__ __align__(16) char lds[];
   __shared__ PzSpShared SS;
   __shared__ AttnShared A;
@@ -424,6 +427,7 @@ int launch_row(pz_sampler* s, const float* d_in, long ld_in, float* d_out, long 
   if (nsw <= 1) return launch_row_t<1>(s, d_in, ld_in, d_out, ld_out, n_rows, n, d_len, nc, lds);
   if (nsw <= 2) return launch_row_t<2>(s, d_in, ld_in, d_out, ld_out, n_rows, n, d_len, nc, lds);
   if (nsw <= 4) return launch_row_t<4>(s, d_in, ld_in, d_out, ld_out, n_rows, n, d_len, nc, lds);
+  static_assert(AR_SEGS <= 8 * AR_WAVES, "the longest row fits the last form");
   return launch_row_t<8>(s, d_in, ld_in, d_out, ld_out, n_rows, n, d_len, nc, lds);
 }
 

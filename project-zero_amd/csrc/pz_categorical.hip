@@ -252,6 +252,7 @@ struct CatEstP {
 // LDS): the exact normaliser.  pen_bytes: the row's penalty tables, then the
 // walk's arrays.
 constexpr int CAT_WALK_BLOCK = 512;
+static_assert(pz_sp_walk_block_ok(CAT_WALK_BLOCK), "");
 template <bool VEC>
 __global__ __launch_bounds__(CAT_WALK_BLOCK) void k_cat_walk(CatArgs A, int pen_bytes) {
   extern __shared__ __align__(16) char lds[];

@@ -193,6 +193,7 @@ __global__ __launch_bounds__(PZ_SP_BLOCK) PZ_SP_TWO_PER_CU void k_spec_rec(SpecA
 // 512 threads: one wave walks, the others stage and pre-evaluate, and two
 // workgroups share a CU with room for the walk's registers.
 constexpr int SPEC_WALK_BLOCK = 512;
+static_assert(pz_sp_walk_block_ok(SPEC_WALK_BLOCK), "");
 template <bool VEC>
 __global__ __launch_bounds__(SPEC_WALK_BLOCK) void k_spec_walk(SpecArgs A) {
   extern __shared__ __align__(16) char lds[];

@@ -855,6 +855,17 @@ inline int pz_sp_walk_nc(int nseg, size_t max_lds) {
   return 0;
 }
 
+// Block sizes the walk's set-up works for: whole waves, a walker and at least
+// one producer, at most as many waves as PzSpShared has totals for (red,
+// red2, list) and at least a thread per ring slot.  (The passes over a slice
+// -- pz_sp_stat_slice, pz_sp_prefix, pz_sp_predict, pz_sp_records,
+// pz_sp_front -- take PZ_SP_BLOCK threads and nothing else: their strides and
+// reductions are PZ_SP_WAVES waves.)
+constexpr bool pz_sp_walk_block_ok(int block) {
+  return block % 64 == 0 && block >= 128 && block <= PZ_SP_BLOCK && PZ_SP_WAVES <= PZ_SP_NC &&
+         PZ_SP_NC <= 64;
+}
+
 // The walk's state is wave-uniform; saying so lets the compiler keep it in
 // scalar registers and branch on it with scalar instructions.
 __device__ __forceinline__ void pz_sp_uni(PzAcc& st) {
