@@ -632,9 +632,9 @@ def run_lm_head(args, torch, cpu):
             s.h, dw, V, n, dx, B, n, dl, V)] * steps)
         t_fu = events_ms(torch, s.stream, [lambda: s.lib.pz_lm_head_argmax_bf16(
             s.h, dw, V, n, dx, B, n, di)] * steps)
-        # batch 4 and up: the matrix-core kernel, one weight pass per 32 rows;
+        # batch 4 and up: the matrix-core kernel, one weight pass per 256 rows;
         # below, the vector kernel's single tile
-        passes = -(-B // 32) if B >= 4 else 1
+        passes = -(-B // 256) if B >= 4 else 1
         b_un = passes * V * n * 2 + B * n * 4 + B * V * 4
         b_fu = passes * V * n * 2 + B * n * 4 + B * 4
         e = {"batch": B, "weight_passes": passes,

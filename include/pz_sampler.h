@@ -316,8 +316,12 @@ PZ_API int pz_softmax_batch(pz_sampler *s, const float *d_in, long ld_in, float 
  * int32 [n_rows], or NULL for len_r = n); d_out[r, 0 .. len_r) receives the
  * probabilities, bit-identical to the reference, and entries from len_r on
  * are not written (a row with len_r <= 0 is left alone).  d_in and d_out may
- * be the same buffer.  Rows of up to 4096 scores run one wave each, longer
- * ones one workgroup each.  Asynchronous on the sampler's stream. */
+ * be the same buffer.  n of up to 1024, and of up to 4096 with more rows than
+ * a round or two of workgroups, runs one wave per row, up to 8192 one
+ * workgroup per row, and longer rows are split over workgroups (whose
+ * workspace the first such call, and one with more or longer rows, allocates
+ * after waiting for the stream).  Asynchronous on the sampler's stream
+ * otherwise. */
 PZ_API int pz_attn_softmax(pz_sampler *s, const float *d_in, long ld_in, float *d_out,
                            long ld_out, int n_rows, int n, const int32_t *d_len);
 
@@ -329,8 +333,11 @@ PZ_API int pz_attn_softmax(pz_sampler *s, const float *d_in, long ld_in, float *
  * wcls; d_x: device [B, ldx] fp32 final-norm activations; fp32
  * accumulation.  The summation order is not the reference's SIMD order, so
  * logits equal the exact product to fp32 rounding (|error| <= n * 2^-24 *
- * sum_j |w_ij x_bj|), not bit for bit.  B <= max_batch; n * 4 bytes must fit
- * in 96 KiB (n <= 24576).  Asynchronous on the sampler's stream. */
+ * sum_j |w_ij x_bj|), not bit for bit.  For B >= 4, 16-byte aligned d_w and n
+ * a multiple of 8, a logit depends on its row of d_w and its activations
+ * alone, so equal rows give equal logits, in any batch.  B <= max_batch; for
+ * B < 4, other n and other d_w, n * 4 bytes must fit in 96 KiB (n <= 24576).
+ * Asynchronous on the sampler's stream. */
 PZ_API int pz_lm_head_bf16(pz_sampler *s, const uint16_t *d_w, int V, int n,
                            const float *d_x, int B, long ldx, float *d_logits, long ld);
 

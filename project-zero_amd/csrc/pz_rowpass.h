@@ -437,8 +437,8 @@ __device__ __forceinline__ float pz_fast_exp(float d) {
 // (11.1), log2(e)'s rounding 0.22 |d|, v_exp_f32's ulp 2, the roundings of
 // expf, of p = e * inv and of the last product 1 each: 16.1 + 0.22 |d|, and
 // there |d| < 0.7 (170 - g).  eps is twice that; checked on every fp32 d in
-// [-104, 0] at every grid that puts t there, and for random inv.  Below 0.25
-// the term rounds to 0 whatever the error.
+// [-104, 0] at every grid that puts t there, and for five inv from 2^-18 to 1.
+// Below 0.25 the term rounds to 0 whatever the error.
 struct PzIncScale {
   float k, mul, eps;
   bool low;  // a grid below 2^-100 (only at the very start of a row): no estimate

@@ -241,9 +241,10 @@ def test_cutoff_inside_the_first_segment_of_a_long_list(torch_cuda):
 
 @pytest.mark.parametrize("B", [70, 300])
 def test_many_rows_in_the_fallback(torch_cuda, B):
-    """Every row's nucleus is past the gather, in more rows than fit one round
-    of the fallback's sort slots (one per CU): each slot sorts several rows
-    one after the other."""
+    """Every row's nucleus is past the gather: 70 rows with a sort slot each,
+    and 300 rows on 256 slots (one per CU), where a slot sorts a second row
+    after its first.  (Many rows per slot: three slots for every batch of
+    tests/test_zz_no_alloc.py.)"""
     V = 15000
     x = pz.synth_normal(B, V, 0.3, 0xFB)
     u = pz.synth_draws(B, 0xFC)
