@@ -124,13 +124,15 @@ extern "C" int pz_sampler_create(pz_sampler** out, int max_batch, int max_vocab,
     return bail(PZ_EDEVICE);
   s->res_params = new (std::nothrow) pz_row_params_dev[B];
   if (!s->res_params) return bail(PZ_ENOMEM);
-  size_t free_bytes = 0, total_bytes = 0;
-  if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) return bail(PZ_EDEVICE);
+  const int want_slots = max_batch < s->n_cu ? max_batch : s->n_cu;
+  size_t free_bytes = 0, total_bytes = 0;  // (asked for where it decides)
+  if (want_slots > PZ_FB_SLOTS && hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess)
+    return bail(PZ_EDEVICE);
   auto scratch_bytes = [&](int slots) {
     return pz_scratch_layout(max_batch, max_vocab, slots, nullptr, nullptr);
   };
   const int slots = pz_take_slots(
-      max_batch < s->n_cu ? max_batch : s->n_cu, PZ_FB_SLOTS, free_bytes, scratch_bytes,
+      want_slots, PZ_FB_SLOTS, free_bytes, scratch_bytes,
       [&](int n) {
         s->scratch_bytes = scratch_bytes(n);
         if (hipMalloc(&s->d_scratch, s->scratch_bytes) == hipSuccess) return true;
