@@ -9,7 +9,10 @@
 // stream: the draw (k_step_draw, one thread per row), the batched sampler
 // reading the uniforms it wrote, and the EOS flags (k_step_eos).  Batches of
 // one kind need fewer: greedy rows draw nothing, categorical rows draw in
-// their first launch, and both write the flags with the ids.
+// their first launch, and both write the flags with the ids.  Batches of
+// several kinds have no one launch that sees every row, and whether a top-p
+// row draws depends on its first value, which its slices' workgroups would
+// each have to form; those and top-k batches keep all three.
 #include <hip/hip_runtime.h>
 
 #include <string.h>

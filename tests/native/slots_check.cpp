@@ -22,6 +22,7 @@ int main() {
       {"plenty", 256, 4 * MiB, 288 * GiB, 288 * GiB, 256, 1},
       {"a batch below one per CU", 70, 4 * MiB, 288 * GiB, 288 * GiB, 70, 1},
       {"a nearly full device", 256, 4 * MiB, 8 * GiB, 8 * GiB, 32, 1},
+      {"a nearly full device, want between", 70, 4 * MiB, 8 * GiB, 8 * GiB, 32, 1},
       {"half of it fits a 64th", 256, 4 * MiB, 40 * GiB, 40 * GiB, 128, 1},
       {"one allocation fails", 256, 4 * MiB, 288 * GiB, 600 * MiB, 128, 2},
       {"less than 32 fit", 256, 4 * MiB, 100 * MiB, 100 * MiB, 16, 2},
